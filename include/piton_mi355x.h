@@ -194,6 +194,21 @@ PITON_API int32_t piton_mi355x_attn_decode(const float *q, const float *k, const
                                  int64_t stride_oh, int64_t n_keys, int64_t batch, int64_t n_heads,
                                  int32_t head_dim, void *stream);
 
+/* piton_mi355x_attn_decode with the keys of each (batch, head) split over several workgroups whose
+ * partial results meet in `workspace` (device memory, workspace_floats floats, contents
+ * irrelevant before and after; a call in flight needs its own). piton_mi355x_attn_decode_workspace
+ * gives the floats a call of this shape uses, 0 where it does not split; a null or smaller
+ * workspace runs the unsplit kernel. Equal to piton_mi355x_attn_decode to rounding, and the same
+ * call otherwise. No reference counterpart. */
+PITON_API int32_t piton_mi355x_attn_decode_workspace(int64_t n_keys, int64_t batch, int64_t n_heads,
+                                           int32_t head_dim, int64_t *floats);
+PITON_API int32_t piton_mi355x_attn_decode_split(const float *q, const float *k, const float *v, float *out,
+                                       float sm_scale, int64_t stride_qb, int64_t stride_qh, int64_t stride_kb,
+                                       int64_t stride_kh, int64_t stride_kn, int64_t stride_vb,
+                                       int64_t stride_vh, int64_t stride_vn, int64_t stride_ob,
+                                       int64_t stride_oh, int64_t n_keys, int64_t batch, int64_t n_heads,
+                                       int32_t head_dim, float *workspace, int64_t workspace_floats, void *stream);
+
 /* A decode step of one decoder layer in one launch: for each sequence b < batch, the new row
  * LN(x[b]) W + bias (LN as in piton_mi355x_linear_ln, W [d_model, 3 d_model] row-major, bias
  * nullable) is written to cache row (n_keys - 1) * batch + b (q | k | v, each d_model wide, row

@@ -840,117 +840,154 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs g) {
     }
 }
 
-// Short caches (n_keys <= 256, head_dim <= 64: a decoder with a small context): the same
-// arithmetic in the same order as attn_decode_kernel, so the two give identical bits, but every
-// K and V element the workgroup needs is requested before any of it is used: one memory round
-// trip instead of one per key chunk plus a chain of V loads behind the softmax.
-constexpr int kShortDecodeKeys = 256;
-#ifndef PITON_DECODE_SHORT
-#define PITON_DECODE_SHORT 1
-#endif
+// The cache in chunks of DCH keys, one workgroup per (batch, head) and chunk: workgroup (bh, c)
+// attends head bh's query to the keys of chunk c. A single chunk stores the output; several leave
+// (m, l, O) unnormalised in the caller's workspace and attn_decode_merge adds them. Bound by HBM:
+// attn_decode_kernel's one workgroup per head is a serial chain of key loads (64 heads x 4096
+// keys of 64: 64 of 256 CUs, 160 us, 0.84 TB/s); the chunks fill the chip and each workgroup
+// requests its 64 KB of K and V before it uses any of it (25 us, 5.4 TB/s with the merge; 6.3
+// TB/s at 256 heads x 4000 keys).
+//   * D/4 consecutive lanes share a row of K or V, one float4 each, so that a wave's load covers
+//     whole cache lines (16 of a key's dims per lane in four loads, attn_decode_kernel's way,
+//     touches every line eight times: 33 us, and 46 with nontemporal loads);
+//   * lane group kg scores the keys i * KG + kg it also adds to P V, so the weights never leave
+//     its registers; a key's dot product adds over the group by lane exchanges;
+//   * the chunk is sized so that a thread holds 16 float4 of K and 16 of V whatever D is;
+//   * keys past n_keys load the last key's row (in bounds for any strides) and drop out by a score
+//     of -inf and a zeroed V, so an infinity in that row counts once.
+template <int D>
+constexpr int kDecodeChunk = 16384 / D;
 
 template <int D, bool VEC>
-__global__ __launch_bounds__(256) void attn_decode_short(DecodeArgs g) {
-    keep_decode_args(g);
-    static_assert(D <= 64, "short decode holds K and V in registers for head_dim <= 64");
-    __shared__ float p[kShortDecodeKeys];
+__global__ __launch_bounds__(256) void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
+    constexpr int DCH = kDecodeChunk<D>, LPR = D / 4, KG = 256 / LPR, NR = DCH / KG;
+    static_assert(NR == 16, "16 float4 of K and of V per thread");
     __shared__ float red[8];
-    __shared__ float part[256];
-    constexpr int TPK = D / 16, KPP = 256 / TPK, KG = 256 / D;
-    constexpr int NIT = kShortDecodeKeys / KPP, NV = kShortDecodeKeys / KG;
+    __shared__ __attribute__((aligned(16))) float part[KG][D];
     const int t = threadIdx.x;
-    const int64_t bh = blockIdx.x, b = bh / g.n_heads, h = bh % g.n_heads;
-    const float *qp = g.q + b * g.s_qb + h * g.s_qh;
-    const float *kp = g.k + b * g.s_kb + h * g.s_kh;
-    const float *vp = g.v + b * g.s_vb + h * g.s_vh;
-    const int n_keys = g.n_keys, head_dim = g.head_dim;
-    const int sub = t % TPK, kslot = t / TPK, d0 = 16 * sub;
-    const bool dims_ok = d0 < head_dim;
-    const int d = t % D, kg = t / D;
-    const bool d_ok = d < head_dim;
+    const int nbh = gridDim.x / nsplit, bh = blockIdx.x % nbh, chunk = blockIdx.x / nbh;
+    const int64_t b = bh / g.n_heads, h = bh % g.n_heads;
+    const int key0 = chunk * DCH, n = min(DCH, g.n_keys - key0);
+    const int dq = t % LPR, kg = t / LPR;
+    const bool d_ok = 4 * dq < g.head_dim;  // head_dim is a multiple of 16
+    const int d0 = d_ok ? 4 * dq : 0;
+    const float *qp = g.q + b * g.s_qb + h * g.s_qh + d0;
+    const float *kp = g.k + b * g.s_kb + h * g.s_kh + d0;
+    const float *vp = g.v + b * g.s_vb + h * g.s_vh + d0;
+    keep_decode_args(g);
     PITON_PHASE_VARS;
     PITON_PHASE(0);
 
-    f32x4 kv[NIT][4];
+    auto row4 = [](const float *r) {
+        if constexpr (VEC) return __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(r));
+        else return f32x4{r[0], r[1], r[2], r[3]};
+    };
+    f32x4 kv[NR], vv[NR];
+    f32x4 q4 = f32x4{qp[0], qp[1], qp[2], qp[3]};
 #pragma unroll
-    for (int it = 0; it < NIT; it++) {
-        const int j = it * KPP + kslot;
-        const float *kr = kp + (int64_t)j * g.s_kn + d0;
+    for (int i = 0; i < NR; i++) kv[i] = row4(kp + (int64_t)(key0 + min(i * KG + kg, n - 1)) * g.s_kn);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            f32x4 f = {0.f, 0.f, 0.f, 0.f};
-            if (j < n_keys && dims_ok) {
-                if constexpr (VEC) f = *reinterpret_cast<const f32x4 *>(kr + 4 * c);
-                else f = f32x4{kr[4 * c], kr[4 * c + 1], kr[4 * c + 2], kr[4 * c + 3]};
-            }
-            kv[it][c] = f;
-        }
-    }
-    // V through a descriptor bounded at the last key's row: rows past it read as zeros, so the
-    // loads need no per-key predicate. The whole offset is the per-lane one (the descriptor's
-    // range check does not cover `soffset`); the host checks it fits 31 bits.
-    const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(vp), (short)0,
-                                                      (int)(((int64_t)(n_keys - 1) * g.s_vn + head_dim) * 4), 0x00020000);
-    const int vo = (int)((d + (int64_t)kg * g.s_vn) * 4), vstep = (int)(KG * g.s_vn * 4);
-    float vv[NV];
+    for (int i = 0; i < NR; i++) vv[i] = row4(vp + (int64_t)(key0 + min(i * KG + kg, n - 1)) * g.s_vn);
 #pragma unroll
-    for (int i = 0; i < NV; i++)
-        vv[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo + i * vstep, 0, 0));
-    float q16[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) q16[i] = dims_ok ? qp[d0 + i] * g.scale : 0.f;
+    for (int e = 0; e < 4; e++) q4[e] = d_ok ? q4[e] * g.scale : 0.f;
 
     PITON_PHASE_WAIT_LOADS();
     PITON_PHASE(1);
-    float mloc = -INFINITY;
+    float sc[NR], mloc = -INFINITY;
 #pragma unroll
-    for (int it = 0; it < NIT; it++) {
-        const int j = it * KPP + kslot;
-        float sc = 0.f;
-        if (j < n_keys && dims_ok) {
+    for (int i = 0; i < NR; i++) {
+        float s = 0.f;
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                sc = fmaf(q16[4 * c], kv[it][c][0], sc);
-                sc = fmaf(q16[4 * c + 1], kv[it][c][1], sc);
-                sc = fmaf(q16[4 * c + 2], kv[it][c][2], sc);
-                sc = fmaf(q16[4 * c + 3], kv[it][c][3], sc);
-            }
-        }
-#pragma unroll
-        for (int o = 1; o < TPK; o <<= 1) sc += __shfl_xor(sc, o);
-        if (j < n_keys) {
-            if (sub == 0) p[j] = sc;
-            mloc = fmaxf(mloc, sc);
-        }
+        for (int e = 0; e < 4; e++) s = d_ok ? fmaf(q4[e], kv[i][e], s) : 0.f;
+        s += dpp_f<DPP_QUAD_XOR1>(s);
+        s += dpp_f<DPP_QUAD_XOR2>(s);
+        s += dpp_f<DPP_ROW_HALF_MIRROR>(s);
+        if constexpr (LPR >= 16) s += dpp_f<DPP_ROW_MIRROR>(s);
+        if constexpr (LPR >= 32) s += __shfl_xor(s, 16);
+        sc[i] = i * KG + kg < n ? s : -INFINITY;
+        mloc = fmaxf(mloc, sc[i]);
     }
-    for (int j = n_keys + t; j < kShortDecodeKeys; j += 256) p[j] = 0.f;  // weights of absent keys
     const float m = block_reduce4(mloc, MaxOp(), red);
     PITON_PHASE(2);
+    const float mref = m == -INFINITY ? 0.f : m;  // a chunk of -inf scores alone: every weight 0
     float lsum = 0.f;
-    for (int j = t; j < n_keys; j += 256) {
-        const float e = __builtin_amdgcn_exp2f(p[j] - m);
-        p[j] = e;
-        lsum += e;
-    }
-    const float inv = 1.0f / block_reduce4(lsum, SumOp(), red + 4);
-
-    // keys past n_keys add fmaf(+0, +0, acc) = acc (acc starts at +0 and never becomes -0), so
-    // the sum equals attn_decode_kernel's, which skips them
-    float acc = 0.f;
-    if (d_ok) {
 #pragma unroll
-        for (int i = 0; i < NV; i++) acc = fmaf(p[kg + KG * i], vv[i], acc);
+    for (int i = 0; i < NR; i++) {
+        sc[i] = __builtin_amdgcn_exp2f(sc[i] - mref);
+        lsum += sc[i];
     }
-    part[t] = acc;
-    __syncthreads();
-    if (t < D && t < head_dim) {
-        float v = part[t];
+    if (n < DCH)
 #pragma unroll
-        for (int w = 1; w < KG; w++) v += part[w * D + t];
-        g.o[b * g.s_ob + h * g.s_oh + t] = v * inv;
+        for (int i = 0; i < NR; i++)
+            if (i * KG + kg >= n) vv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NR; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] = fmaf(sc[i], vv[i][e], acc[e]);
+    *reinterpret_cast<f32x4 *>(&part[kg][4 * dq]) = acc;
+    const float l = block_reduce4(dq == 0 ? lsum : 0.f, SumOp(), red + 4);  // its barrier publishes the sums
+    float v = 0.f;
+    if (t < D) {
+        v = part[0][t];
+#pragma unroll
+        for (int w = 1; w < KG; w++) v += part[w][t];
+    }
+    if (nsplit == 1) {
+        // (every score -inf: 0 / 0, NaN as the softmax of such a row is)
+        if (t < D && t < g.head_dim) g.o[b * g.s_ob + h * g.s_oh + t] = v * (1.0f / l);
+    } else {
+        float *wp = ws + ((int64_t)bh * nsplit + chunk) * (D + 2);
+        if (t < D) wp[t] = v;
+        if (t == 255) {  // a thread that stores no sum
+            wp[D] = m;
+            wp[D + 1] = l;
+        }
     }
     PITON_PHASE(3);
-    PITON_PHASE_END(kPhaseAttnDecodeShort, g.phase);
+    PITON_PHASE_END(kPhaseAttnDecodePart, g.phase);
+}
+
+// out = sum_c 2^(m_c - M) O_c / sum_c 2^(m_c - M) l_c over the parts of one (batch, head); 256/D
+// groups of threads take the parts c = group mod 256/D and add through LDS in group order.
+template <int D>
+__global__ __launch_bounds__(256) void attn_decode_merge(DecodeArgs g, const float *ws, int nsplit) {
+    constexpr int KG = 256 / D;
+    static_assert(kMaxDecodeKeys / kDecodeChunk<D> <= 64, "one lane per part");
+    __shared__ float wgt[64];
+    __shared__ float part[256];
+    const int t = threadIdx.x, lane = t & 63, d = t % D, kg = t / D;
+    const int64_t bh = blockIdx.x, b = bh / g.n_heads, h = bh % g.n_heads;
+    const float *wp = ws + bh * nsplit * (D + 2);
+    const int c0 = min(lane, nsplit - 1);
+    const float mc = wp[c0 * (D + 2) + D], lc = wp[c0 * (D + 2) + D + 1];
+    const float m = wave_reduce(mc, MaxOp());
+    const float w = lane < nsplit ? __builtin_amdgcn_exp2f(mc - m) : 0.f;
+    const float inv = 1.0f / wave_reduce(lane < nsplit ? w * lc : 0.f, SumOp());
+    if (t < 64) wgt[t] = w;
+    __syncthreads();
+    float acc = 0.f;
+#pragma unroll 8
+    for (int c = kg; c < nsplit; c += KG) acc = fmaf(wgt[c], wp[c * (D + 2) + d], acc);
+    part[t] = acc;
+    __syncthreads();
+    if (t < D && t < g.head_dim) {
+        float v = part[t];
+#pragma unroll
+        for (int k = 1; k < KG; k++) v += part[k * D + t];
+        g.o[b * g.s_ob + h * g.s_oh + t] = v * inv;
+    }
+}
+
+// The chunks of a decode attention call's cache; more than one needs a workspace of
+// decode_workspace() floats. Splitting wins at every head count measured: 8 heads x 4096 keys
+// 155 -> 9 us, 1024 heads x 512 keys (enough workgroups to fill the chip unsplit) 53 -> 46 us.
+static int decode_parts(int64_t n_keys, int32_t head_dim) {
+    const int chunk = head_dim <= 32 ? kDecodeChunk<32> : head_dim == 64 ? kDecodeChunk<64> : kDecodeChunk<128>;
+    return (int)((n_keys + chunk - 1) / chunk);
+}
+static int64_t decode_workspace(int64_t nbh, int parts, int32_t head_dim) {
+    return sat_mul(sat_mul(nbh, parts), (head_dim < 32 ? 32 : head_dim) + 2);
 }
 
 static int attn_launch(AttnArgs g, int64_t batch, int64_t n_heads, int32_t head_dim, hipStream_t st) {
@@ -1054,6 +1091,33 @@ int32_t piton_mi355x_attn_decode(const float *q, const float *k, const float *v,
                                  int64_t stride_kn, int64_t stride_vb, int64_t stride_vh, int64_t stride_vn,
                                  int64_t stride_ob, int64_t stride_oh, int64_t n_keys, int64_t batch, int64_t n_heads,
                                  int32_t head_dim, void *stream) {
+    return piton_mi355x_attn_decode_split(q, k, v, out, sm_scale, stride_qb, stride_qh, stride_kb, stride_kh, stride_kn,
+                                          stride_vb, stride_vh, stride_vn, stride_ob, stride_oh, n_keys, batch, n_heads,
+                                          head_dim, nullptr, 0, stream);
+}
+
+int32_t piton_mi355x_attn_decode_workspace(int64_t n_keys, int64_t batch, int64_t n_heads, int32_t head_dim,
+                                           int64_t *floats) {
+    using namespace piton;
+    PITON_REQUIRE(floats != nullptr, PITON_EINVAL, "attn_decode_workspace: null output");
+    *floats = 0;
+    int rc = require_device();
+    if (rc) return rc;
+    if (n_keys >= 1 && n_keys <= kMaxDecodeKeys && batch > 0 && n_heads > 0) {
+        const int parts = decode_parts(n_keys, head_dim);
+        const int64_t nbh = sat_mul(batch, n_heads);
+        if (parts > 1 && sat_mul(nbh, parts) <= 0x7FFFFFFF) *floats = decode_workspace(nbh, parts, head_dim);
+    }
+    clear_error();
+    return PITON_OK;
+}
+
+int32_t piton_mi355x_attn_decode_split(const float *q, const float *k, const float *v, float *out, float sm_scale,
+                                       int64_t stride_qb, int64_t stride_qh, int64_t stride_kb, int64_t stride_kh,
+                                       int64_t stride_kn, int64_t stride_vb, int64_t stride_vh, int64_t stride_vn,
+                                       int64_t stride_ob, int64_t stride_oh, int64_t n_keys, int64_t batch,
+                                       int64_t n_heads, int32_t head_dim, float *workspace, int64_t workspace_floats,
+                                       void *stream) {
     using namespace piton;
     PITON_REQUIRE(n_keys >= 1 && batch >= 0 && n_heads >= 0, PITON_EINVAL, "attn_decode: n_keys=%lld batch=%lld",
                   (long long)n_keys, (long long)batch);
@@ -1072,17 +1136,31 @@ int32_t piton_mi355x_attn_decode(const float *q, const float *k, const float *v,
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)(batch * n_heads)), block(256);
     const bool vec = aligned16(k) && stride_kn % 4 == 0 && stride_kh % 4 == 0 && stride_kb % 4 == 0;
+    const int parts = decode_parts(n_keys, head_dim);
+    if (parts == 1 || (workspace && sat_mul(batch * n_heads, parts) <= 0x7FFFFFFF &&
+                       workspace_floats >= decode_workspace(batch * n_heads, parts, head_dim))) {
+        const bool vec4 = vec && aligned16(v) && stride_vn % 4 == 0 && stride_vh % 4 == 0 && stride_vb % 4 == 0;
+        const dim3 pgrid((unsigned)(batch * n_heads * parts));
+#define PITON_DEC_SPLIT(D)                                                                                          \
+    do {                                                                                                            \
+        if (vec4) PITON_LAUNCH((attn_decode_part<D, true>), pgrid, block, 0, st, g, workspace, parts);              \
+        else PITON_LAUNCH((attn_decode_part<D, false>), pgrid, block, 0, st, g, workspace, parts);                  \
+        if (parts > 1) PITON_LAUNCH((attn_decode_merge<D>), grid, block, 0, st, g, workspace, parts);                            \
+    } while (0)
+        if (head_dim <= 32) PITON_DEC_SPLIT(32);
+        else if (head_dim == 64) PITON_DEC_SPLIT(64);
+        else PITON_DEC_SPLIT(128);
+#undef PITON_DEC_SPLIT
+        rc = check_launch("attn_decode");
+        if (rc == PITON_OK) clear_error();
+        return rc;
+    }
 #define PITON_DEC(KERNEL, D)                                                                                        \
     do {                                                                                                            \
         if (vec) PITON_LAUNCH((KERNEL<D, true>), grid, block, 0, st, g);                                      \
         else PITON_LAUNCH((KERNEL<D, false>), grid, block, 0, st, g);                                         \
     } while (0)
-    // short caches: every V offset the kernel forms (up to 256 rows and 64 dims) within 31 bits
-    const bool short_cache = PITON_DECODE_SHORT && n_keys <= kShortDecodeKeys && stride_vn >= 0 &&
-                             ((int64_t)kShortDecodeKeys * stride_vn + 64) * 4 < 0x7FFFFFFF;
-    if (head_dim <= 32 && short_cache) PITON_DEC(attn_decode_short, 32);
-    else if (head_dim == 64 && short_cache) PITON_DEC(attn_decode_short, 64);
-    else if (head_dim <= 32) PITON_DEC(attn_decode_kernel, 32);
+    if (head_dim <= 32) PITON_DEC(attn_decode_kernel, 32);
     else if (head_dim == 64) PITON_DEC(attn_decode_kernel, 64);
     else PITON_DEC(attn_decode_kernel, 128);
 #undef PITON_DEC

@@ -100,7 +100,7 @@ static inline PhaseRecord *phase_slot() { return nullptr; }
 #define PITON_PHASE_TU(name)
 #endif
 // kernel ids of the trace records
-constexpr uint32_t kPhaseSoftmaxRows = 1, kPhaseSoftmaxWg = 2, kPhaseAttnFast = 3, kPhaseAttnDecodeShort = 4,
+constexpr uint32_t kPhaseSoftmaxRows = 1, kPhaseSoftmaxWg = 2, kPhaseAttnFast = 3, kPhaseAttnDecodePart = 4,
                    kPhaseDecodeLayer = 5, kPhaseMlp = 6, kPhaseGemmSplit = 7;
 
 // numpy's argmax rule on (value, index) pairs: a NaN beats any number, the larger value beats

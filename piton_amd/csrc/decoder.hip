@@ -26,7 +26,7 @@
 //     a branch whose join waits for it); and the barriers wait for LDS work only (__syncthreads
 //     would also wait for the copies and for the cache-row store);
 //   * the new q, k, v go to the cache row (t = n_keys - 1) and to LDS, and the attention runs
-//     as attn_decode_short does: TPK = 4 lanes per key score 16 dims each (read from LDS in a
+//     the way attn_decode_kernel does: TPK = 4 lanes per key score 16 dims each (read from LDS in a
 //     bank-conflict-free chunk order), the maximum and the sum of 2^(s - m) reduce over the
 //     workgroup, thread (d, g) sums p_j V[j][d] over the keys j = g (mod 8) in key order, and
 //     the eight partial sums add in order.

@@ -62,6 +62,8 @@ SIGNATURES = {
     "piton_mi355x_mlp3": [_p, _i64] + [_p] * 6 + [_i64] * 4 + [_p, _p, _i32, _p],
     "piton_mi355x_attn_fwd_batched": [_p, _p, _p, _p, _f32] + [_i64] * 16 + [_i32, _i32, _p],
     "piton_mi355x_attn_decode": [_p, _p, _p, _p, _f32] + [_i64] * 13 + [_i32, _p],
+    "piton_mi355x_attn_decode_workspace": [_i64, _i64, _i64, _i32, ctypes.POINTER(_i64)],
+    "piton_mi355x_attn_decode_split": [_p, _p, _p, _p, _f32] + [_i64] * 13 + [_i32, _p, _i64, _p],
     "piton_mi355x_decode_layer": [_p, _i64, _f32, _p, _p, _p, _i64, _p, _i64, _f32, _i64, _i64, _i64, _i32, _i64,
                                   _p, _p, _p, _i64, _p, _p],
     "piton_mi355x_lm_head_argmax": [_p, _i64, _f32, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i32, _p],
@@ -333,13 +335,34 @@ def attn_fwd_batched(q, k, v, out, sm_scale, s_qb, s_qh, s_qm, s_kb, s_kh, s_kn,
 
 def attn_decode(q, k, v, out, sm_scale, s_qb, s_qh, s_kb, s_kh, s_kn, s_vb, s_vh, s_vn, s_ob, s_oh, n_keys, batch,
                 heads, head_dim):
-    """One query per (batch, head) against n_keys cached keys."""
+    """One query per (batch, head) against n_keys cached keys (long caches split over the keys
+    through a workspace from torch's allocator, which keeps it for the current stream)."""
     check_tensor("q", q, max_offset=_span((batch, s_qb), (heads, s_qh), (head_dim, 1)))
     check_tensor("k", k, max_offset=_span((batch, s_kb), (heads, s_kh), (n_keys, s_kn), (head_dim, 1)))
     check_tensor("v", v, max_offset=_span((batch, s_vb), (heads, s_vh), (n_keys, s_vn), (head_dim, 1)))
     check_tensor("out", out, max_offset=_span((batch, s_ob), (heads, s_oh), (head_dim, 1)))
-    _call("piton_mi355x_attn_decode", _ptr(q), _ptr(k), _ptr(v), _ptr(out), float(sm_scale), s_qb, s_qh, s_kb, s_kh,
-          s_kn, s_vb, s_vh, s_vn, s_ob, s_oh, n_keys, batch, heads, int(head_dim), _stream())
+    args = (_ptr(q), _ptr(k), _ptr(v), _ptr(out), float(sm_scale), s_qb, s_qh, s_kb, s_kh, s_kn, s_vb, s_vh, s_vn, s_ob,
+            s_oh, n_keys, batch, heads, int(head_dim))
+    # a cache of one chunk (16384 / head_dim keys) needs no workspace
+    ws = _decode_workspace(n_keys, batch, heads, int(head_dim)) if n_keys > 16384 // max(int(head_dim), 32) else None
+    if ws is None:
+        _call("piton_mi355x_attn_decode", *args, _stream())
+    else:
+        _call("piton_mi355x_attn_decode_split", *args, _ptr(ws), ws.numel(), _stream())
+
+
+
+def _decode_workspace(n_keys, batch, heads, head_dim):
+    """The split decode attention's workspace, or None where the call does not split (or the
+    device has no memory left for it: the unsplit kernel needs none)."""
+    n = _i64(0)
+    _call("piton_mi355x_attn_decode_workspace", n_keys, batch, heads, head_dim, ctypes.byref(n))
+    if n.value == 0:
+        return None
+    try:
+        return torch.empty(n.value, device="cuda")
+    except torch.OutOfMemoryError:
+        return None
 
 
 def decode_layer(x, ldx, eps, w, bias, cache, ldc, out, ldo, sm_scale, n_keys, batch, heads, head_dim, d_model,
