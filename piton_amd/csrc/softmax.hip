@@ -5,8 +5,8 @@
 //     (max, then sum), and written once: 8 bytes of HBM traffic per element, the minimum;
 //   * rows of up to 1024 columns: one 64-lane wavefront per row, four per 256-thread
 //     workgroup, reductions by DPP lane moves only (no LDS, no barriers);
-//   * rows of up to 16K columns: one 256-thread workgroup per row, reductions by DPP within
-//     each wave and then through LDS across the four. Many short-lived workgroups keep reads
+//   * rows of up to 64K columns: one workgroup per row (256 or 512 threads up to 16K columns,
+//     1024 above), reductions by DPP within each wave and then through LDS across them. Many short-lived workgroups keep reads
 //     and writes interleaved across the chip; at 4096 x 4096 this streams ~8 % faster than
 //     a single generation of row-per-wave waves, which read together and then write together;
 //   * loads and stores are nontemporal: the row is touched once. (Cached loads look faster
@@ -23,8 +23,8 @@
 //     entry gives exactly 0 and the rest of the row is a normal softmax, as in the emulator,
 //     whose fmax orders -NaN lowest and whose float ALUs read it as -inf
 //     (piton/qpu/emulator.py:139-147, 173-177, 201-205, 224-225); numpy makes that row NaN;
-//   * longer rows take a workgroup-per-row kernel that reads the row three times (max, sum,
-//     write).
+//   * longer rows take a workgroup-per-row kernel that reads the row twice (maximum and sum
+//     together, then the write).
 #include "common.h"
 
 // kernel per row class (float4 chunks per lane: short <= 4, mid 5..8, long 9..16):
@@ -97,8 +97,10 @@ __device__ __forceinline__ float row_reduce(float v, Op op, float *red) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) red[wave] = v;
     __syncthreads();
-    if (T == 256) return op(op(red[0], red[1]), op(red[2], red[3]));
-    return op(op(op(red[0], red[1]), op(red[2], red[3])), op(op(red[4], red[5]), op(red[6], red[7])));
+    auto four = [&](int w) { return op(op(red[w], red[w + 1]), op(red[w + 2], red[w + 3])); };
+    if constexpr (T == 256) return four(0);
+    else if constexpr (T == 512) return op(four(0), four(4));
+    else return op(op(four(0), four(4)), op(four(8), four(12)));
 }
 
 // Masks row `row` (held in b, window offset off) to [0, n), normalises it and stores it.
@@ -211,9 +213,12 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(float *out, const flo
     PITON_PHASE_END(kPhaseSoftmaxRows, phase);
 }
 
-// One T-thread workgroup per row (T = 256 or 512, CH chunks per thread): many short-lived
+// One T-thread workgroup per row (T = 256, 512 or 1024, CH chunks per thread): many short-lived
 // workgroups keep the chip's reads and writes interleaved, which streams faster than a single
-// generation of row-per-wave waves.
+// generation of row-per-wave waves. Rows of 16K to 64K columns fill the registers of 1024
+// threads (a row is read once: 512 x 50000 207 -> 39.6 us, 5.2 TB/s; 1000 x 32000 155 -> 45.2 us,
+// 5.7 TB/s; the three passes of a 256-thread workgroup before). 512 threads with twice the
+// chunks measured the same (39.6, 46.2 us).
 template <int CH, int T, bool ALIGNED>
 __global__ __launch_bounds__(T) void softmax_wg_kernel(float *out, const float *in, int64_t in_rs, int64_t out_rs,
                                                        int n, PhaseRecord *phase) {
@@ -230,32 +235,77 @@ __global__ __launch_bounds__(T) void softmax_wg_kernel(float *out, const float *
     PITON_PHASE_END(kPhaseSoftmaxWg, phase);
 }
 
-// Rows too long for registers: one workgroup per row, three passes over the row.
-__device__ __forceinline__ float block_reduce(float v, float *red, bool is_max) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    v = is_max ? wave_reduce(v, MaxOp()) : wave_reduce(v, SumOp());
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    float r = red[0];
-    for (int w = 1; w < 4; w++) r = is_max ? fmaxf(r, red[w]) : r + red[w];
-    __syncthreads();
-    return r;
-}
+// Rows too long for registers (over 64K columns): one 1024-thread workgroup per row, two passes
+// over it (200 x 100000 378 -> 42 us, 64 x 250000 924 -> 53 us against three scalar passes of
+// 256 threads; with fewer rows than CUs bound by what one CU streams). Each thread keeps a
+// running maximum and the sum of exps under it (rescaled where the maximum moves, at most once
+// per LCH chunks), which merge across the workgroup; then the row is read again (from the
+// last-level cache where it fits), normalised and stored.
+constexpr int LT = 1024, LCH = 8;
 
-__global__ __launch_bounds__(256) void softmax_long_kernel(float *out, const float *in, int64_t in_rs, int64_t out_rs,
-                                                           int64_t n) {
-    __shared__ float red[4];
+template <bool ALIGNED>
+__global__ __launch_bounds__(LT) void softmax_long_kernel(float *out, const float *in, int64_t in_rs, int64_t out_rs,
+                                                          int64_t n) {
+    __shared__ float red[2 * LT / 64];
     const int64_t row = blockIdx.x;
     const float *rp = in + row * in_rs;
     float *op = out + row * out_rs;
-    float mx = -INFINITY;
-    for (int64_t i = threadIdx.x; i < n; i += 256) mx = fmaxf(mx, rp[i]);
-    const float m = block_reduce(mx, red, true);
-    float s = 0.f;
-    for (int64_t i = threadIdx.x; i < n; i += 256) s += exp_row(qpu_neg_nan(rp[i]) - m);
-    s = block_reduce(s, red, false);
+    // the aligned float4 window covering the row, as in load_row; LCH * LT chunks at a time
+    const int off = ALIGNED ? 0 : (int)((reinterpret_cast<uintptr_t>(rp) >> 2) & 3);
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(rp - off);
+    const int64_t nch = (off + n + 3) >> 2;
+    auto load = [&](f32x4 (&b)[LCH], int64_t c0) {
+#pragma unroll
+        for (int c = 0; c < LCH; c++) {
+            const int64_t ci = c0 + threadIdx.x + LT * c;
+            b[c] = src[ci < nch ? ci : nch - 1];
+        }
+#pragma unroll
+        for (int c = 0; c < LCH; c++) {
+            const int64_t e0 = 4 * (c0 + threadIdx.x + LT * c) - off;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (!(e0 + j >= 0 && e0 + j < n)) b[c][j] = -INFINITY;
+        }
+    };
+    float m = -INFINITY, s = 0.f;
+    for (int64_t c0 = 0; c0 < nch; c0 += LCH * LT) {
+        f32x4 b[LCH];
+        load(b, c0);
+        float mx = m;
+#pragma unroll
+        for (int c = 0; c < LCH; c++) mx = fmaxf(mx, fmaxf(fmaxf(b[c].x, b[c].y), fmaxf(b[c].z, b[c].w)));
+        // (nothing above -inf so far: the terms are 0 under a reference of 0)
+        const float ref = mx == -INFINITY ? 0.f : mx;
+        s *= exp_row((m == -INFINITY ? ref : m) - ref);
+        m = mx;
+#pragma unroll
+        for (int c = 0; c < LCH; c++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) s += exp_row(qpu_neg_nan(b[c][j]) - ref);
+    }
+    const float mr = row_reduce<LT>(m, MaxOp(), red);
+    // a thread without a value above -inf adds its sum (0, or NaN from a NaN entry) as it is
+    s = row_reduce<LT>(m == -INFINITY ? s : s * exp_row(m - mr), SumOp(), red + LT / 64);
     const float inv = 1.0f / s;
-    for (int64_t i = threadIdx.x; i < n; i += 256) op[i] = exp_row(qpu_neg_nan(rp[i]) - m) * inv;
+    const bool vec = ALIGNED || (int)((reinterpret_cast<uintptr_t>(op) >> 2) & 3) == off;
+    for (int64_t c0 = 0; c0 < nch; c0 += LCH * LT) {
+        f32x4 b[LCH];
+        load(b, c0);
+#pragma unroll
+        for (int c = 0; c < LCH; c++) {
+            const int64_t e0 = 4 * (c0 + threadIdx.x + LT * c) - off;
+#pragma unroll
+            for (int j = 0; j < 4; j++) b[c][j] = exp_row(qpu_neg_nan(b[c][j]) - mr) * inv;
+            if (vec && e0 >= 0 && e0 + 3 < n) {
+                __builtin_nontemporal_store(b[c], reinterpret_cast<f32x4 *>(op + e0));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (e0 + j >= 0 && e0 + j < n) op[e0 + j] = b[c][j];
+            }
+        }
+    }
 }
 
 // Launches the wave-per-row kernel: one row per wave (mode 0), or persistent waves, as many
@@ -308,7 +358,6 @@ extern "C" int32_t piton_mi355x_softmax(float *out, const float *in, int64_t in_
     const bool all_aligned = aligned16(in) && (in_row_stride % 4 == 0 || n_rows == 1);
     const int64_t nch = (n + 3 + (all_aligned ? 0 : 3)) / 4;
     const int64_t per_lane = (nch + 63) / 64;
-    const dim3 block(256);
     const bool aligned = aligned16(in) && aligned16(out) && n % 4 == 0 &&
                          ((in_row_stride % 4 == 0 && out_row_stride % 4 == 0) || n_rows == 1);
     const int mode = per_lane <= 4 ? PITON_SM_SHORT : per_lane <= 8 ? PITON_SM_MID : per_lane <= 16 ? PITON_SM_LONG : 2;
@@ -340,8 +389,13 @@ extern "C" int32_t piton_mi355x_softmax(float *out, const float *in, int64_t in_
     else if (per_lane <= 16) PITON_SM_WG(PITON_SM_LONG_CH, 64 * PITON_SM_LONG_CH == 256 ? 256 : 512);
     else if (per_lane <= 32) PITON_SM_WG(8, 256);
     else if (per_lane <= 64) PITON_SM_WG(16, 256);
+    else if (per_lane <= 128) PITON_SM_WG(8, 1024);
+    else if (per_lane <= 256) PITON_SM_WG(16, 1024);
+    else if (aligned)
+        PITON_LAUNCH((softmax_long_kernel<true>), dim3((unsigned)n_rows), dim3(LT), 0, st, out, in, in_row_stride,
+                           out_row_stride, n);
     else
-        PITON_LAUNCH(softmax_long_kernel, dim3((unsigned)n_rows), block, 0, st, out, in, in_row_stride,
+        PITON_LAUNCH((softmax_long_kernel<false>), dim3((unsigned)n_rows), dim3(LT), 0, st, out, in, in_row_stride,
                            out_row_stride, n);
 #undef PITON_SM_WG
 #undef PITON_SM
