@@ -23,7 +23,9 @@
 //   * causal: a query group visits only the key blocks up to its last query, only blocks that
 //     can hold a masked key are masked, and each XCD issues its longest groups first;
 //   * K is read through (stride_kn, stride_kk): float4 along d for [N, D] storage, scalar
-//     loads (consecutive keys across lanes) for pre-transposed [D, N] storage.
+//     loads (consecutive keys across lanes) for pre-transposed [D, N] storage;
+//   * aligned shapes of head_dim 32, 64 and 128 take a pipelined kernel with the same arithmetic
+//     (attn_fwd_fast, attn_fwd_fast_dn, below).
 #include "common.h"
 
 #include <algorithm>
@@ -383,8 +385,11 @@ __device__ __forceinline__ f32x4 bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) 
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
 }
 
-// The fast kernel: head_dim == D, Q / K / V / O rows contiguous and 16-byte aligned (K in
-// [N, D] order), every row offset of a head within 2^31 bytes (checked on the host). Per query
+// The fast kernel: head_dim == D, Q / K / V / O rows contiguous and 16-byte aligned (or K stored
+// [D, N], of any alignment: KDN), every row offset of a head within 2^31 bytes (checked on the host).
+// MFMA-bound: 73 us for 32 x 1024 x 64 (117 TFLOP/s of 156), 268 us for 16 x 2000 x 128 (122; the
+// general kernel 408), 44.2 us for 32 x 1024 x 64 causal with K [D, N] (97 as with K [N, D]; the
+// general kernel's guarded scalar K loads 190 us). Per query
 // group it runs the general kernel's blocks and arithmetic (wave w takes key blocks
 // first_block(w, qg), + ANW, ..., the same online softmax and the same merge formula), so the two
 // agree bit for bit:
@@ -394,7 +399,10 @@ __device__ __forceinline__ f32x4 bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) 
 //   * Q' (pre-scaled) is staged once per workgroup in LDS. The paired kernel (two waves per
 //     SIMD) loads a wave's B operand of the score product into 32 registers per group, so the
 //     product is MFMAs alone; the single-group kernel (three waves per SIMD, no registers to
-//     spare) keeps Q' transposed (qT[d][query]) and reads the operand per step, conflict-free;
+//     spare) keeps Q' transposed (qT[d][query]) and reads the operand per step, conflict-free, and
+//     so does D = 128 (two waves per SIMD: O, one K block and two score blocks fill 230 of 256);
+//   * KDN loads one float per dim and lane, consecutive keys across the lanes (whole 128-byte lines
+//     per half wave), where [N, D] rows load 16 bytes of a key per lane;
 //   * V blocks are copied from memory straight into the wave's LDS slab (16-byte LDS-DMA);
 //   * software pipeline: block j+1's score product is issued beside block j's exps, K is loaded
 //     two blocks ahead and V one block ahead; Q is requested first and the first block's K
@@ -406,6 +414,8 @@ __device__ __forceinline__ f32x4 bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) 
 #ifndef PITON_ATTN_FAST_WAVES
 #define PITON_ATTN_FAST_WAVES 3
 #endif
+// waves per SIMD the fast kernel is register-budgeted for
+constexpr int fast_waves(int d, bool pair) { return pair || d > 64 ? 2 : PITON_ATTN_FAST_WAVES; }
 // causal query groups in pairs: 0 never, 1 always, 2 when the pairs fill at most two
 // workgroups per CU (one generation)
 #ifndef PITON_ATTN_PAIR_MODE
@@ -501,10 +511,10 @@ __device__ __forceinline__ void merge_quarter(const float (*xo)[D / 2][64], cons
     }
 }
 
-template <int D, bool PAIR>
-__global__ __launch_bounds__(64 * ANW) __attribute__((amdgpu_waves_per_eu(PAIR ? 2 : PITON_ATTN_FAST_WAVES)))
-void attn_fwd_fast(AttnArgs g) {
+template <int D, bool PAIR, bool KDN>
+__device__ __forceinline__ void fast_body(AttnArgs g) {
     constexpr int NG = PAIR ? 2 : 1;
+    static_assert(!PAIR || D <= 64, "a pair of 128-wide groups exceeds the registers and the LDS of two waves per SIMD");
     // Two LDS objects. The V slabs (written by LDS-DMA) and the Q tiles are distinct variables,
     // so the compiler's wait-count pass can tell the Q reads of a score product from the V
     // copies in flight and does not make them wait for those copies. The merge reuses both: each
@@ -513,11 +523,11 @@ void attn_fwd_fast(AttnArgs g) {
     constexpr int QT_F = NG * D * AQG, XM_F = NG * ANW * 2 * 64;
     __shared__ __attribute__((aligned(16))) float lds_v[SLAB_F > XO_F ? SLAB_F : XO_F];
     __shared__ __attribute__((aligned(16))) float lds_q[QT_F > XM_F ? QT_F : XM_F];
-    static_assert(!PAIR || sizeof(lds_v) + sizeof(lds_q) <= 80 * 1024, "two paired workgroups share a CU's 160 KB");
+    static_assert(sizeof(lds_v) + sizeof(lds_q) <= 80 * 1024, "two workgroups share a CU's 160 KB");
     float(*vslab)[ABN][D] = reinterpret_cast<float(*)[ABN][D]>(lds_v);
     // the Q' tiles: row-major and swizzled (q2) when the operand is loaded into registers once
     // per group, transposed (qT) when every score product reads it
-    constexpr bool QREG = PAIR || PITON_ATTN_FAST_WAVES <= 2;
+    constexpr bool QREG = D <= 64 && fast_waves(D, PAIR) <= 2;
     float(*q2)[AQG][D] = reinterpret_cast<float(*)[AQG][D]>(lds_q);
     float(*qT)[D][AQG] = reinterpret_cast<float(*)[D][AQG]>(lds_q);
 
@@ -540,7 +550,10 @@ void attn_fwd_fast(AttnArgs g) {
     const int n_ctx = (int)g.n_ctx;
     const uint32_t s_qm = (uint32_t)g.s_qm, s_kn = (uint32_t)g.s_kn, s_vn = (uint32_t)g.s_vn;
     const auto rq = make_rsrc(g.q + bi * g.s_qb + h * g.s_qh, ((uint32_t)(n_ctx - 1) * s_qm + D) * 4u);
-    const auto rk = make_rsrc(g.k + bi * g.s_kb + h * g.s_kh, ((uint32_t)(n_ctx - 1) * s_kn + D) * 4u);
+    // (KDN: K stored [D, N], keys contiguous, dims s_kk apart)
+    const uint32_t s_kk = KDN ? (uint32_t)g.s_kk : 1u;
+    const auto rk = make_rsrc(g.k + bi * g.s_kb + h * g.s_kh,
+                              KDN ? ((uint32_t)(D - 1) * s_kk + n_ctx) * 4u : ((uint32_t)(n_ctx - 1) * s_kn + D) * 4u);
     const auto rv = make_rsrc(g.v + bi * g.s_vb + h * g.s_vh, ((uint32_t)(n_ctx - 1) * s_vn + D) * 4u);
 
     // this wave's blocks: list index j < n0 is block f0 + ANW*j of the first group, j >= n0
@@ -556,13 +569,31 @@ void attn_fwd_fast(AttnArgs g) {
     // byte offsets: K half row of key kb*32 + l31; V chunk c of block kb at v_lane + kb*v_blk + c*v_c
     constexpr int KPC = 64 / (D / 4);  // V keys per float4 chunk step of the lane
     constexpr int NVQ = ABN * D / 4 / 64;
-    constexpr int K_LOADS = D / 8;  // 16-byte loads of load_k: one lane-half row of the block
+    // loads of load_k: a lane-half row of the block in 16-byte pieces, or (KDN) one float per dim
+    // (a count past the 63 that vmcnt holds only makes its wait the stricter one)
+    constexpr int K_LOADS = KDN ? (D / 2 < 63 ? D / 2 : 63) : D / 8;
     static_assert(K_LOADS <= 63 && NVQ <= 63, "loads per block within the vmcnt range");
-    const uint32_t k_lane = ((uint32_t)l31 * s_kn + half * (D / 2)) * 4u, k_blk = (uint32_t)ABN * s_kn * 4u;
+    const uint32_t k_lane = KDN ? half * (D / 2) * s_kk * 4u : ((uint32_t)l31 * s_kn + half * (D / 2)) * 4u;
+    const uint32_t k_blk = (uint32_t)ABN * s_kn * 4u;
     const uint32_t v_lane = ((uint32_t)(lane / (D / 4)) * s_vn + 4 * (lane % (D / 4))) * 4u;
     const uint32_t v_blk = (uint32_t)ABN * s_vn * 4u, v_c = (uint32_t)KPC * s_vn * 4u;
     float(*vw)[D] = vslab[wave];
     auto load_k = [&](float (&kf)[D / 2], int kb) {
+        if constexpr (KDN) {
+            // consecutive keys across the lanes, one dim per load and half; a key past the last
+            // reads the last (in bounds for every dim) and is masked with the block's scores
+            const uint32_t off = k_lane + (uint32_t)min(kb * ABN + l31, n_ctx - 1) * 4u;
+            // (the dims' offsets from a zero the compiler cannot see through: known, it holds all
+            // D/2 of them in scalar registers across the loop and spills)
+            int dim = 0;
+            asm volatile("" : "+s"(dim));
+#pragma unroll
+            for (int s = 0; s < D / 2; s++) {
+                kf[s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, (int)off, dim, 0));
+                dim += (int)(s_kk * 4u);
+            }
+            return;
+        }
         const uint32_t off = k_lane + (uint32_t)kb * k_blk;
 #pragma unroll
         for (int c = 0; c < D / 8; c++) {
@@ -640,7 +671,21 @@ void attn_fwd_fast(AttnArgs g) {
         float qf[D / 2];
         // (a wave can hold no block of the first group and some of the second)
         if constexpr (QREG) load_q_operand<D>(qf, q2[PAIR && n0 == 0 ? 1 : 0], half, l31);
-        auto scores = [&]() { return QREG ? block_scores<D>(kf, qf) : block_scores_lds<D>(kf, qT[0], half, l31); };
+        auto scores = [&]() {
+            if constexpr (KDN) {
+                // holds the operand in groups of four consecutive registers, where the score product
+                // waits for it: left to itself, the compiler gives the loop's separate loads a
+                // second set of registers and spills
+#pragma unroll
+                for (int c = 0; c < D / 8; c++) {
+                    f32x4 f = {kf[4 * c], kf[4 * c + 1], kf[4 * c + 2], kf[4 * c + 3]};
+                    asm volatile("" : "+v"(f));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) kf[4 * c + e] = f[e];
+                }
+            }
+            return QREG ? block_scores<D>(kf, qf) : block_scores_lds<D>(kf, qT[0], half, l31);
+        };
         f32x16 st = scores();
         // Every pass of the loop starts with block j+1's K in flight ahead of block j's V, so
         // the wait for that K lets the newer V copies stay in flight. Block 0's V is therefore
@@ -662,6 +707,8 @@ void attn_fwd_fast(AttnArgs g) {
                 st_next = scores();
             }
             online_exp(st, mref, l_i);
+            // (KDN: its many loads, moved up into the score product, would need a second operand set)
+            if constexpr (NEXT && KDN) __builtin_amdgcn_sched_barrier(0);
             if constexpr (NEXT) load_k(kf, kb_of(j + 2));
             // block j's V is in the slab once at most the K loads just issued (D / 8 of them) are
             // in flight (vmcnt counts in issue order; the scheduling barriers keep that order)
@@ -725,6 +772,18 @@ void attn_fwd_fast(AttnArgs g) {
     }
     PITON_PHASE(3);
     PITON_PHASE_END(kPhaseAttnFast, g.phase);
+}
+
+template <int D, bool PAIR>
+__global__ __launch_bounds__(64 * ANW) __attribute__((amdgpu_waves_per_eu(fast_waves(D, PAIR))))
+void attn_fwd_fast(AttnArgs g) {
+    fast_body<D, PAIR, false>(g);
+}
+// K stored [D, N]
+template <int D, bool PAIR>
+__global__ __launch_bounds__(64 * ANW) __attribute__((amdgpu_waves_per_eu(fast_waves(D, PAIR))))
+void attn_fwd_fast_dn(AttnArgs g) {
+    fast_body<D, PAIR, true>(g);
 }
 
 template <int D>
@@ -999,27 +1058,38 @@ static int attn_launch(AttnArgs g, int64_t batch, int64_t n_heads, int32_t head_
     g.nbh = (int)(batch * n_heads);
     g.phase = phase_slot();
     dim3 grid((unsigned)((int64_t)g.nqg * g.nbh));
-    // the fast kernel: exact head_dim, contiguous aligned rows that do not overlap, and every
-    // byte offset it forms (rows up to n_ctx + 3 * ANW * 32, the loads a few blocks past the
-    // end included) within 31 bits
-    const int64_t smax = std::max(g.s_qm, std::max(g.s_kn, g.s_vn));
-    const bool fast = (head_dim == 32 || head_dim == 64) && kl == K_VEC_D && g.q_vec && g.v_vec &&
+    // the fast kernel: exact head_dim, contiguous aligned rows that do not overlap (or K stored
+    // [D, N]: keys contiguous, dims any distance apart), and every byte offset it forms (rows up to
+    // n_ctx + 3 * ANW * 32, the loads a few blocks past the end included) within 31 bits
+    const bool kdn = kl != K_VEC_D && g.s_kn == 1 && g.s_kk > 0;
+    const int64_t smax = std::max(g.s_qm, std::max(kdn ? 1 : g.s_kn, g.s_vn));
+    const bool k_fast = kdn ? sat_mul(sat_add(sat_mul(head_dim, g.s_kk), g.n_ctx), 4) < (1LL << 31)
+                            : kl == K_VEC_D && g.s_kn >= head_dim;
+    const bool fast = (head_dim == 32 || head_dim == 64 || head_dim == 128) && k_fast && g.q_vec && g.v_vec &&
                       aligned16(g.o) && g.s_om % 4 == 0 && g.s_oh % 4 == 0 && g.s_ob % 4 == 0 &&
-                      g.s_qm >= head_dim && g.s_kn >= head_dim && g.s_vn >= head_dim &&
+                      g.s_qm >= head_dim && g.s_vn >= head_dim &&
                       ((g.n_ctx + 3 * ANW * ABN + AQG) * smax + head_dim) * 4 < (1LL << 31);
     bool pair = false;
-    if (fast && g.causal && g.nqg > 1) {
+    if (fast && head_dim <= 64 && g.causal && g.nqg > 1) {
         const int64_t pairs = (int64_t)g.nbh * ((g.nqg + 1) / 2);
         pair = PITON_ATTN_PAIR_MODE == 1 || (PITON_ATTN_PAIR_MODE == 2 && pairs <= 2 * (int64_t)device_cu_count());
         if (pair) grid = dim3((unsigned)pairs);
     }
-    if (fast && head_dim == 64) {
-        if (pair) PITON_LAUNCH((attn_fwd_fast<64, true>), grid, dim3(64 * ANW), 0, st, g);
-        else PITON_LAUNCH((attn_fwd_fast<64, false>), grid, dim3(64 * ANW), 0, st, g);
-    } else if (fast) {
-        if (pair) PITON_LAUNCH((attn_fwd_fast<32, true>), grid, dim3(64 * ANW), 0, st, g);
-        else PITON_LAUNCH((attn_fwd_fast<32, false>), grid, dim3(64 * ANW), 0, st, g);
-    }
+#define PITON_ATTN_FAST(D, PAIR)                                                                                    \
+    do {                                                                                                            \
+        if (kdn)                                                                                                    \
+            PITON_LAUNCH_NAMED((attn_fwd_fast_dn<D, PAIR>), "attn_fwd_fast_dn<" #D ", " #PAIR ">", grid,            \
+                               dim3(64 * ANW), 0, st, g);                                                           \
+        else                                                                                                        \
+            PITON_LAUNCH_NAMED((attn_fwd_fast<D, PAIR>), "attn_fwd_fast<" #D ", " #PAIR ">", grid, dim3(64 * ANW),  \
+                               0, st, g);                                                                           \
+    } while (0)
+    if (fast && head_dim == 128) PITON_ATTN_FAST(128, false);
+    else if (fast && head_dim == 64 && pair) PITON_ATTN_FAST(64, true);
+    else if (fast && head_dim == 64) PITON_ATTN_FAST(64, false);
+    else if (fast && pair) PITON_ATTN_FAST(32, true);
+    else if (fast) PITON_ATTN_FAST(32, false);
+#undef PITON_ATTN_FAST
     else if (head_dim <= 32) launch_d<32>(kl, g, grid, st);
     else if (head_dim == 64) launch_d<64>(kl, g, grid, st);
     else launch_d<128>(kl, g, grid, st);
