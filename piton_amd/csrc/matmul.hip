@@ -18,6 +18,7 @@
 //     so the stored elements equal sum_k A[m,k] B[k,n] exactly as the reference's masks give;
 //   * tile order: workgroups renumbered so each XCD gets a contiguous run of logical ids,
 //     then the reference's GROUP_SIZE_M grouping (kernels.py:28-36) on those ids.
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -518,21 +519,23 @@ void gemm_direct_kernel(GemmArgs g) {
         }
 }
 
-// Shapes with too few 128 x 128 tiles to fill the chip (config 2's 512^3 has 16 and 1024^3 64
-// for 256 CUs) or with ragged edges: a workgroup owns a 32 NB x 32 NBN tile and its KS waves
-// split K, each wave computing the whole tile, NB x NBN blocks of v_mfma_f32_32x32x2_f32, over
-// the K tiles kt = wave, wave + KS, ... (interleaved, so the waves read neighbouring k together).
+// Shapes that are not whole generations of the direct kernel's tiles: few tiles (512^3 has 16 of
+// 128 x 128 for 256 CUs, 1024^3 64), ragged edges, a last generation part full. A workgroup owns a
+// 32 NB x 32 NBN tile and its KS waves split K, each wave computing the whole tile, NB x NBN blocks
+// of v_mfma_f32_32x32x2_f32, over the K tiles kt = wave, wave + KS, ... (interleaved, so the waves
+// read neighbouring k together); kSplitForms lists the forms and plan_split chooses. 64 x 128 tiles
+// with one wave over K run as the direct kernel's wide form does (one wave per SIMD, 4000^3 0.90 of
+// the matrix rate; 0.73 with 64 x 64 tiles at several waves per SIMD and masks in the loop).
 // Operands go from memory straight into registers as in the direct kernel (the same k order
 // inside a K tile of 32: lane half h supplies k = 16 h + s at step s), through buffer
 // descriptors bounded at each matrix's last element. The K tail (k >= K inside the last tile,
-// which may hold padding or the next row or column) reads as zeros, as the reference's K mask
-// makes it: a row-major A's values there are masked (16-byte chunks by their offset, an
-// unaligned row's values after its shift), a column-major B's chunks take an offset past the
-// bound; a column-major A's elements (columns at least M floats apart) and a row-major B's rows
-// past K (rows at least N floats apart) lie past the bound already. Rows of A past M and columns
-// of B past N feed only rows and columns of C that are not stored. The KS partial tiles meet in
-// LDS and add in wave order (fixed: the result does not depend on timing); the epilogue (bias,
-// ReLU, residual) then stores rows < M and columns < N.
+// which may hold padding or the next row or column) adds zeros, as the reference's K mask makes
+// it: it is multiplied apart from the whole tiles, the values of a row-major A and a column-major B
+// masked in registers; a column-major A's elements (columns at least M floats apart) and a
+// row-major B's rows past K (rows at least N floats apart) lie past the bound and read as zeros.
+// Rows of A past M and columns of B past N feed only rows and columns of C that are not stored. The
+// KS partial tiles meet in LDS and add in wave order (fixed: the result does not depend on timing);
+// the epilogue (bias, ReLU, residual) then stores rows < M and columns < N.
 // AM: A's layout. A_ROW16: row-major, rows 16-byte aligned (16-byte loads along k). A_ROW:
 // row-major, each lane's 16 consecutive A values sit r = (row start) mod 4 floats past a 16-byte
 // boundary, the same r for every K tile: the lane loads the five aligned 16-byte chunks that
@@ -540,35 +543,20 @@ void gemm_direct_kernel(GemmArgs g) {
 // instead of 16 loads). A_COL: column-major (stride 1 along M), one float per k, coalesced over
 // the lanes' 32 rows. BKC: B column-major (stride 1 along K, 16-byte aligned, K % 4 == 0),
 // 16-byte loads along k; otherwise B has stride 1 along N and loads one float per k.
-#ifndef PITON_SPLIT_MAX_WAVES
-#define PITON_SPLIT_MAX_WAVES 4
-#endif
-#ifndef PITON_SPLIT_WAVES_PER_CU
-#define PITON_SPLIT_WAVES_PER_CU 8
-#endif
-// the wide 64 x 128 tile of the split kernel (0: square tiles only)
-#ifndef PITON_SPLIT_WIDE
-#define PITON_SPLIT_WIDE 1
-#endif
-// the direct kernel takes whole-tile shapes with at least this many 128 x 128 tiles per CU
 // grids with more tiles than CUs run as one launch per generation of one tile per CU (0: one
 // launch of the multi-workgroup kernel, PITON_GEMM_DIRECT_WAVES workgroups per CU)
 #ifndef PITON_GEMM_GEN_LAUNCHES
 #define PITON_GEMM_GEN_LAUNCHES 1
 #endif
-#ifndef PITON_DIRECT_TILES_PER_CU
-#define PITON_DIRECT_TILES_PER_CU 1
-#endif
-constexpr int kMaxSplitWaves = PITON_SPLIT_MAX_WAVES;
 enum SplitA { A_ROW16 = 0, A_ROW = 1, A_COL = 2 };
-
 template <int NB, int NBN, int KS, int AM, bool BKC, bool TAIL>
-__global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
+__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(1, KS == 1 && NBN == 4 ? 1 : 8)))
+void gemm_split_kernel(GemmArgs g) {
     constexpr bool AVEC = AM == A_ROW16;
     constexpr int TB = 32 * NB, TBN = 32 * NBN;  // tile rows and columns
     constexpr int NACC = NB * NBN * 16;          // accumulator registers per lane
     // the partial tiles: [wave][group of four accumulators][lane], 16 bytes per lane and group
-    __shared__ f32x4 red[KS > 1 ? KS : 1][NACC / 4][64];
+    __shared__ f32x4 red[KS > 1 ? KS : 1][KS > 1 ? NACC / 4 : 1][64];
     keep_epilogue_args(g);
     // the wave index is uniform: readfirstlane makes the K loop, which starts at it, a scalar loop
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
@@ -600,27 +588,36 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
     const int64_t a_end = off0 + (g.M - 1) * s_am + (g.K - 1) * s_ak + 1;  // floats from a_al
     const int64_t a_bound = ((a_end + 3) & ~(int64_t)3) * 4;                              // bytes
     const int64_t b_bound = ((g.K - 1) * s_bk + (g.N - 1) * s_bn + 1) * 4;
+    // per-lane offsets that do not change from tile to tile. An operand that loads one float per k
+    // (a column-major A, a row-major B) keeps an offset per k, its blocks 128 bytes apart in the
+    // instructions' immediate offsets; on tiles 128 columns wide, which leave no registers for
+    // those, an offset per block and the k of a whole tile in the scalar offset, which the range
+    // check does not cover: there rows (columns) past the edge are the last one (they feed only
+    // elements that are not stored). The scalar offsets on 64 x 64 tiles measured slower: 1024^3
+    // 21.7 -> 23.5 us.
+    constexpr bool KSOFF = NBN == 4;
     uint32_t va[NB], vb[NBN];
     int ra_shift[NB];  // A_ROW: this lane's row start past its 16-byte boundary, in floats
 #pragma unroll
     for (int i = 0; i < NB; i++) {
-        const int64_t e0 = off0 + (m0 + i * 32 + l31) * s_am + 16 * half * s_ak;
+        const int64_t m = m0 + i * 32 + l31;
+        const int64_t e0 = off0 + (AM == A_COL && KSOFF ? min(m, g.M - 1) : m) * s_am + 16 * half * s_ak;
         ra_shift[i] = (int)(e0 & 3);
         va[i] = (uint32_t)((AM == A_COL ? e0 : e0 & ~(int64_t)3) * 4);
     }
 #pragma unroll
-    for (int j = 0; j < NBN; j++) vb[j] = (uint32_t)(((int64_t)(16 * half) * s_bk + (n0 + j * 32 + l31) * s_bn) * 4);
+    for (int j = 0; j < NBN; j++) {
+        const int64_t n = n0 + j * 32 + l31;
+        vb[j] = (uint32_t)(((int64_t)(16 * half) * s_bk + (!BKC && KSOFF ? min(n, g.N - 1) : n) * s_bn) * 4);
+    }
     const uint32_t sak4 = (uint32_t)(s_ak * 4), sbk4 = (uint32_t)(s_bk * 4);
-    const int nk = (int)((g.K + 31) / 32);
-    // per-lane offsets that do not change from tile to tile: one float per k of a column-major A
-    // (va[i] is va[0] + 128 i) and of a row-major B (vb[j] is vb[0] + 128 j): the block offsets
-    // go in the instructions' immediate offsets
-    uint32_t vas[AM == A_COL ? 16 : 1], vbs[BKC ? 1 : 16];
-    if constexpr (AM == A_COL) {
+    const int nk = (int)(g.K / 32);  // whole K tiles; TAIL: then a partial one
+    uint32_t vas[AM == A_COL && !KSOFF ? 16 : 1], vbs[!BKC && !KSOFF ? 16 : 1];
+    if constexpr (AM == A_COL && !KSOFF) {
 #pragma unroll
         for (int s = 0; s < 16; s++) vas[s] = va[0] + s * sak4;
     }
-    if constexpr (!BKC) {
+    if constexpr (!BKC && !KSOFF) {
 #pragma unroll
         for (int s = 0; s < 16; s++) vbs[s] = vb[0] + s * sbk4;
     }
@@ -631,47 +628,45 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
         float b[NBN][16];
     };
     // A tile's loads go through descriptors whose base is advanced to the tile and whose bound
-    // shrinks by as much (scalar arithmetic only: with K % 32 == 0 the loop has no vector address
-    // arithmetic), so the range check, which covers the per-lane offset, still ends each at its
-    // matrix's last element: offsets at or past it read as zero. Tiles past the last one (a wave's
-    // K tiles come in pairs) read through a bound of 0: zeros. TAIL (K % 32 != 0), inside the
-    // last tile, k >= K: a column-major A's and a row-major B's elements lie past the bound; a
-    // row-major A's 16-byte chunks and a column-major B's get an offset past the bound (2^31) by a
-    // select against the tile's remaining k (a compare and a select per chunk, no branch: control
-    // flow in the loop makes the compiler copy the accumulators out of AGPRs each iteration).
-    constexpr uint32_t kOut = 0x80000000u;
-    auto rsrc = [&](const float *base, int64_t bound, uint32_t step4, int kt) {
+    // shrinks by as much (scalar arithmetic only: the loop has no vector address arithmetic), so
+    // the range check, which covers the per-lane offset, still ends each at its matrix's last
+    // element: offsets at or past it read as zero. Tiles past the last whole one (the loop's
+    // prefetch) read through a bound of 0: zeros. The tail tile adds the k in the per-lane offset:
+    // the k >= K of a column-major A and a row-major B lie past the bound and are zeros; along K the
+    // operand holds the padding or the next row, which `mul` masks.
+    auto rsrc = [&](const float *base, int64_t bound, uint32_t step4, int kt, int end) {
         const int64_t shift = (int64_t)kt * 32 * step4;  // past the last tile the base is never read
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(base) + shift),
-                                                 (short)0, scalar_lt_select(kt, nk, (int)(bound - shift)),
+                                                 (short)0, scalar_lt_select(kt, end, (int)(bound - shift)),
                                                  0x00020000);
     };
     // PIN keeps the loads in source order with scheduling barriers (A first, then B step by step).
-    auto load = [&](int kt, Ops &o, auto pin) {
-        const auto ra = rsrc(a_al, a_bound, sak4, kt);
-        const auto rb = rsrc(g.b, b_bound, sbk4, kt);
-        const int rem = (int)(g.K - (int64_t)kt * 32) - 16 * half;  // TAIL: this lane's k below K in the tile
-        // TAIL: the offset of a chunk of four k starting c past the lane's first k of the tile
-        auto chunk = [&](uint32_t off, int c) -> int { return (int)(!TAIL || c < rem ? off : kOut); };
+    auto load_tile = [&](int kt, Ops &o, auto pin, auto tail) {
+        constexpr bool T = decltype(tail)::value;
+        const auto ra = rsrc(a_al, a_bound, sak4, kt, nk + T);
+        const auto rb = rsrc(g.b, b_bound, sbk4, kt, nk + T);
         auto pinned = [&]() {
             if constexpr (decltype(pin)::value) __builtin_amdgcn_sched_barrier(0);
+        };
+        // k = s of block i: per-lane offsets per k, or per block with the k in the scalar offset
+        auto load_k = [&](auto r, const auto &per_k, const auto &per_block, uint32_t step4, int s, int i) {
+            const int off = (int)(KSOFF ? per_block[i] + (T ? s * step4 : 0u) : per_k[s] + 128 * i);
+            return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, KSOFF && !T ? (int)(s * step4) : 0, 0));
         };
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             if constexpr (AM == A_COL) {
-                // columns no closer than M floats apart (the host checks it): (m, k) with k >= K
-                // lies at or past (K - 1) s_ak + M, the bound
 #pragma unroll
                 for (int s = 0; s < 16; s++) {
-                    o.a[i][s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ra, (int)(vas[s] + 128 * i), 0, 0));
+                    o.a[i][s] = load_k(ra, vas, va, sak4, s, i);
                     pinned();
                 }
             } else {
                 // A_ROW16: four chunks of four k; A_ROW: the five chunks holding k0 - r .. k0 - r + 19
 #pragma unroll
                 for (int q = 0; q < (AVEC ? 4 : 5); q++) {
-                    const int off = AVEC ? chunk(va[i] + 16 * q, 4 * q) : (int)(va[i] + 16 * q);
-                    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, off, 0, 0));
+                    const f32x4 v =
+                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va[i] + 16 * q), 0, 0));
 #pragma unroll
                     for (int e = 0; e < 4; e++) o.a[i][4 * q + e] = v[e];
                     pinned();
@@ -684,7 +679,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const f32x4 v =
-                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, chunk(vb[j] + 16 * q, 4 * q), 0, 0));
+                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(vb[j] + 16 * q), 0, 0));
 #pragma unroll
                     for (int e = 0; e < 4; e++) o.b[j][4 * q + e] = v[e];
                     pinned();
@@ -694,22 +689,29 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
             for (int s = 0; s < 16; s++)
 #pragma unroll
                 for (int j = 0; j < NBN; j++) {
-                    o.b[j][s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rb, (int)(vbs[s] + 128 * j), 0, 0));
+                    o.b[j][s] = load_k(rb, vbs, vb, sbk4, s, j);
                     pinned();
                 }
         }
     };
+    auto load = [&](int kt, Ops &o, auto pin) { load_tile(kt, o, pin, std::false_type()); };
     using Pin = std::true_type;
     using Free = std::false_type;
-    f32x16 acc[NB][NBN];
+    // 64 x 128 and 32 x 32 tiles with one wave over K add even and odd K tiles apart (the registers
+    // are there), so that their sums are no longer chains than two waves over K have: 2500 x 3000 x
+    // 2000 is off float64 by 5.7e-7 so and 8.0e-7 with one chain, at the same speed
+    constexpr int NSUM = KS == 1 && NBN != 2 ? 2 : 1;
+    f32x16 acc[NSUM][NB][NBN];
 #pragma unroll
-    for (int i = 0; i < NB; i++)
+    for (int u = 0; u < NSUM; u++)
 #pragma unroll
-        for (int j = 0; j < NBN; j++)
+        for (int i = 0; i < NB; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-    // A_ROW: the lane's 16 values of block i: window[s + r], zero where k0 + s >= K
-    auto a_vals = [&](const Ops &o, int i, int kt, float (&v)[16]) {
+            for (int j = 0; j < NBN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[u][i][j][r] = 0.f;
+    // A_ROW: the lane's 16 values of block i: window[s + r]
+    auto a_vals = [&](const Ops &o, int i, float (&v)[16]) {
         if constexpr (AM != A_ROW) {
 #pragma unroll
             for (int s = 0; s < 16; s++) v[s] = o.a[i][s];
@@ -717,7 +719,6 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
             // bitwise blends with all-ones / all-zero masks (v_bfi): a select between two array
             // elements becomes a dynamic index, which moves the array to scratch memory
             const int r = ra_shift[i];
-            const int64_t nvalid = g.K - ((int64_t)kt * 32 + 16 * half);
             const uint32_t m1 = 0u - (uint32_t)(r & 1), m2 = 0u - (uint32_t)((r >> 1) & 1);
             uint32_t t0[18];
 #pragma unroll
@@ -727,22 +728,32 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
             }
 #pragma unroll
             for (int s = 0; s < 16; s++) {
-                const uint32_t x = t0[s] ^ ((t0[s] ^ t0[s + 2]) & m2);
-                v[s] = __uint_as_float(x & (0u - (uint32_t)(s < nvalid)));
+                v[s] = __uint_as_float(t0[s] ^ ((t0[s] ^ t0[s + 2]) & m2));
             }
         }
     };
-    auto mul = [&](const Ops &o, int kt) {
+    // MASKED (the K tail): values with k >= K, which the operands along K may hold from the padding
+    // or the next row or column, are zeros
+    auto mul = [&](const Ops &o, f32x16 (&acc)[NB][NBN], int kt, auto masked) {
+        constexpr bool MASKED = decltype(masked)::value;
+        const int rem = (int)(g.K - (int64_t)kt * 32) - 16 * half;  // this lane's k below K in the tile
         float av[NB][16];
 #pragma unroll
-        for (int i = 0; i < NB; i++) a_vals(o, i, kt, av[i]);
+        for (int i = 0; i < NB; i++) {
+            a_vals(o, i, av[i]);
+            if constexpr (MASKED && AM != A_COL)
+#pragma unroll
+                for (int s = 0; s < 16; s++) av[i][s] = s < rem ? av[i][s] : 0.f;
+        }
 #pragma unroll
         for (int s = 0; s < 16; s++)
 #pragma unroll
-            for (int i = 0; i < NB; i++)
+            for (int j = 0; j < NBN; j++) {
+                const float bv = !(MASKED && BKC) || s < rem ? o.b[j][s] : 0.f;
 #pragma unroll
-                for (int j = 0; j < NBN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][s], o.b[j][s], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < NB; i++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][s], bv, acc[i][j], 0, 0, 0);
+            }
     };
     // this wave's K tiles: wave, wave + KS, ...; the next one is in flight while one multiplies.
     // Tiles come in pairs with no condition between loads and products (a conditional product
@@ -795,17 +806,36 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
     if constexpr (PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     PITON_PHASE_WAIT_LOADS();
     PITON_PHASE(1);
-    for (int kt = wave; kt < nk; kt += 2 * KS) {
+    // TAIL, before the loop, which takes pairs of whole tiles: the partial tile, masked (masks inside
+    // the loop, a compare and a select per 16-byte chunk and tile, held 2500 x 3000 x 2000 to 0.72 of
+    // the matrix rate), and the first tile of a wave with an odd count (a zero tile padded the pair).
+    // The kernel without them is kept for K a multiple of 64 KS: the loop behind them measured 1024^3
+    // at 22.5 us against 21.5.
+    int kt = wave;
+    if constexpr (TAIL) {
+        if (wave == nk % KS && g.K % 32 != 0) {
+            load_tile(nk, o1, Free(), std::true_type());
+            mul(o1, acc[0], nk, std::true_type());
+        }
+        if (nk > wave && ((nk - wave + KS - 1) / KS) % 2) {
+            load(kt + KS, o1, Free());
+            mul(o0, acc[NSUM - 1], kt, std::false_type());
+            o0 = o1;
+            kt += KS;
+            if constexpr (PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // as after the prologue's
+        }
+    }
+    for (; kt < nk; kt += 2 * KS) {
         if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         __builtin_amdgcn_sched_barrier(0);
         load(kt + KS, o1, Free());
-        mul(o0, kt);
+        mul(o0, acc[0], kt, std::false_type());
         interleave();
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         __builtin_amdgcn_sched_barrier(0);
         load(kt + 2 * KS, o0, Free());
-        mul(o1, kt + KS);
+        mul(o1, acc[NSUM - 1], kt + KS, std::false_type());
         interleave();
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -827,7 +857,8 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
             for (int j = 0; j < NBN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) store(i, j, r, lane, acc[i][j][r]);
+                for (int r = 0; r < 16; r++)
+                    store(i, j, r, lane, NSUM == 1 ? acc[0][i][j][r] : acc[0][i][j][r] + acc[NSUM - 1][i][j][r]);
     } else {
 #pragma unroll
         for (int i = 0; i < NB; i++)
@@ -836,7 +867,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
                 for (int q = 0; q < 4; q++)
                     red[wave][(i * NBN + j) * 4 + q][lane] =
-                        f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                        f32x4{acc[0][i][j][4 * q], acc[0][i][j][4 * q + 1], acc[0][i][j][4 * q + 2], acc[0][i][j][4 * q + 3]};
         // an LDS-only barrier: the partials are in LDS; nothing here waits for other memory
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -1103,20 +1134,81 @@ static int layout_b(const GemmArgs &g) {
     return SCALAR;
 }
 
-// The split kernel's tile (NB blocks of 32 per side), waves per workgroup and operand layouts
-// for a shape, or nb = 0 when it does not apply. Tiles of 64 when there are at least as many as
-// CUs, else of 32; then the waves double (up to kMaxSplitWaves) until the launch has
-// PITON_SPLIT_WAVES_PER_CU waves per CU, as long as each wave keeps at least two K tiles
-// (8 per CU: 1536^3 103 -> 88 us against 4; the other shapes measured the same).
+// The split kernel's forms (tile of nb x nbn blocks of 32, ks waves over K) with a model of a
+// launch's time in us: t0 + the longer of
+//   * rounds * (products of a wave * stretch + round): the waves go one to a SIMD, where a product
+//     of 32 x 32 x 32 takes 0.432 us (16 MFMAs of 64 clocks at 2.37 GHz);
+//   * the operand bytes the waves load over what the L2s deliver (`mbus`, MB per us), which bounds
+//     the 32 x 32 tiles (half the products per byte of the 64 x 64 ones);
+// each by layout: 16-byte rows, A's rows unaligned, B column-major. Fitted to 78 shapes from 80 x 64
+// x 120 to 2560^3 in every form, three operand sets in turn (4-7 % rms); taking the form it names
+// costs 1.4 % on average against the best one measured. The rule before (tiles of 64 from as many of
+// them as CUs, waves doubled up to eight per CU) cost 6.5 %: 1536^3 82.6 -> 71.1 us, 2697 x 1640 x
+// 2428 233 -> 203, 128 x 340 x 200 6.5 -> 5.5. Two waves over K are left out: the two such
+// workgroups of a CU ran one after the other (1330 x 212 x 3772 57 us against 52 with four).
+// `sums`: the interleaved partial sums of an element's K tiles; forms with as many add alike.
+struct SplitForm {
+    int nb, nbn, ks, sums;
+    float t0, stretch[3], round, mbus[3];
+};
+constexpr SplitForm kSplitForms[] = {
+    {2, 4, 1, 2, 5.2f, {1.02f, 1.09f, 1.02f}, 8.0f, {12.f, 12.f, 12.f}},
+    {2, 2, 1, 1, 3.4f, {1.02f, 1.14f, 1.02f}, 5.8f, {12.f, 12.f, 12.f}},
+    {1, 1, 1, 2, 5.2f, {1.06f, 1.51f, 1.01f}, 0.0f, {12.5f, 10.5f, 10.8f}},
+    {2, 4, 4, 4, 1.2f, {1.04f, 1.12f, 1.07f}, 7.7f, {12.f, 12.f, 12.f}},
+    {2, 2, 4, 4, 4.0f, {1.11f, 1.22f, 1.14f}, 2.4f, {12.f, 12.f, 12.f}},
+    {1, 1, 4, 4, 4.2f, {1.39f, 1.59f, 1.56f}, 0.3f, {19.5f, 10.5f, 10.7f}},
+};
+constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
+constexpr int kSplitWide = 3;  // the index of <2, 4, 4>
+
+static int64_t split_tiles(const SplitForm &f, int64_t M, int64_t N) {
+    return sat_mul((M + 32 * f.nb - 1) / (32 * f.nb), (N + 32 * f.nbn - 1) / (32 * f.nbn));
+}
+constexpr int kAnyLayout = -1;  // the mean of aligned rows and B column-major
+static float split_us(const SplitForm &f, int64_t M, int64_t N, int64_t K, int layout, int cus) {
+    const int64_t slots = 4 * (int64_t)cus / f.ks, nk = (K + 31) / 32;
+    const int64_t tiles = split_tiles(f, M, N);
+    int64_t rounds = (tiles + slots - 1) / slots;
+    // workgroups of one wave where two fit a SIMD: the dispatcher does not spread one round of them
+    // evenly (1023 tiles of 64 x 64 on 1024 SIMDs took 150 or 282 us, depending on what ran before;
+    // as workgroups of four waves with a tile each, full rounds of them took 10 % longer)
+    if (f.ks == 1 && f.nbn < 4 && tiles > 2 * (int64_t)cus && rounds < 2) rounds = 2;
+    const float wave = 0.432f * f.nb * f.nbn * (float)((nk + f.ks - 1) / f.ks);
+    const float mb = (float)tiles * (float)nk * (f.nb + f.nbn) * 4096e-6f;
+    auto us = [&](int l) { return f.t0 + std::max((float)rounds * (wave * f.stretch[l] + f.round), mb / f.mbus[l]); };
+    return layout == kAnyLayout ? 0.5f * (us(0) + us(2)) : us(layout);
+}
+// the fastest form by the model, of those with `sums` partial sums (0: of all)
+static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int sums, float &us) {
+    int best = -1;
+    for (int i = 0; i < kNumSplitForms; i++) {
+        if (sums && kSplitForms[i].sums != sums) continue;
+        const float t = split_us(kSplitForms[i], M, N, K, layout, cus);
+        if (best < 0 || t < us) best = i, us = t;
+    }
+    return best;
+}
+
+// A product as one launch, or as two: whole rounds of one form over the first rows (columns) of C
+// and the rest in the form that suits it, where the model finds that faster than letting a last
+// round run part full (2560^3 296 -> 269 us, 300 x 4000 x 3000 94 -> 73). parts 0: the split
+// kernel does not apply. The cut and the partial sums depend on the sizes alone, so every layout of
+// A and B (and every group order) adds each element's products in the same order and gives the
+// same bits.
+struct SplitPart {
+    int form;
+    int64_t m0, n0, M, N;
+};
 struct SplitPlan {
-    int nb, ks;
-    int64_t tiles;
+    int parts;
+    SplitPart part[2];
     int am;    // SplitA: A's layout
     bool bkc;  // B column-major
-    int nbn;   // blocks of 32 columns per tile (nb, or 2 nb: the wide tile)
+    float us;
 };
 static SplitPlan plan_split(const GemmArgs &g, int cus) {
-    SplitPlan p{0, 0, 0, A_ROW16, false, 0};
+    SplitPlan p{0, {}, 0, false, 0.f};
     if (g.K <= 0 || g.M <= 0 || g.N <= 0) return p;
     // A with stride 1 along K (16-byte loads where its rows are 16-byte aligned and K % 4 == 0) or
     // along M with columns at least M floats apart; B with stride 1 along N and rows at least N
@@ -1129,37 +1221,61 @@ static SplitPlan plan_split(const GemmArgs &g, int cus) {
     if (g.s_bn == 1 && g.s_bk >= g.N) p.bkc = false;
     else if (g.s_bk == 1 && g.s_bn > 0 && g.s_bn % 4 == 0 && g.K % 4 == 0 && aligned16(g.b)) p.bkc = true;
     else return p;
-    auto tiles2 = [&](int64_t tm, int64_t tn) { return sat_mul((g.M + tm - 1) / tm, (g.N + tn - 1) / tn); };
-    auto tiles = [&](int64_t tb) { return tiles2(tb, tb); };
-    const int64_t nk = (g.K + 31) / 32;
-#ifndef PITON_SPLIT_NB_MAX
-#define PITON_SPLIT_NB_MAX 2
-#endif
-    const int nb = PITON_SPLIT_NB_MAX > 1 && tiles(64) >= cus ? 2 : 1;
-    const int64_t nt = tiles(32 * nb);
-    int ks = 1;
-    // (eight waves only on 64 x 64 tiles: their reduction gives each wave two groups of four
-    // accumulators; a 32 x 32 tile has four groups)
-    const int ks_max = nb == 2 ? kMaxSplitWaves : min(kMaxSplitWaves, 4);
-    while (ks < ks_max && nt * ks < PITON_SPLIT_WAVES_PER_CU * (int64_t)cus && 4 * ks <= nk) ks *= 2;
-    // every byte offset a lane forms (the prefetch past the last tile included) stays below 2^31
-    const int64_t tb = 32 * nb, kpad = g.K + 32 * (2 * ks + 3);  // the farthest prefetch: tile nk - 1 + 2 ks
-    if (sat_add(sat_mul(g.M + tb, g.s_am), sat_mul(kpad, g.s_ak)) >= (1LL << 29) - 4 ||
-        sat_add(sat_mul(kpad, g.s_bk), sat_mul(g.N + tb, g.s_bn)) >= (1LL << 29) || nt > 0x7FFFFFFF)
+    // every byte offset a lane forms (edge tiles of up to 128, a tail tile's 31 k) stays below 2^31
+    const int64_t kpad = g.K + 64;
+    if (sat_add(sat_mul(g.M + 128, g.s_am), sat_mul(kpad, g.s_ak)) >= (1LL << 29) - 4 ||
+        sat_add(sat_mul(kpad, g.s_bk), sat_mul(g.N + 128, g.s_bn)) >= (1LL << 29) ||
+        split_tiles(SplitForm{1, 1}, g.M, g.N) > 0x7FFFFFFF)
         return p;
-    p.nb = nb, p.ks = ks, p.tiles = nt, p.nbn = nb;
-    // the wide tile, 64 x 128: where 64 x 64 tiles would put two workgroups on some CUs and the
-    // 64 x 128 ones fit one per CU (the ragged 1000 x 1800 x 700: 464 against 240), four waves
-    // splitting K give each SIMD one wave with the same MFMA work as two waves of the square
-    // tile, and the wave's 2 x 4 blocks need 0.56 loads per product instead of 0.63
-    const int64_t ntw = tiles2(64, 128);
-    // (measured with B row-major: 2048 x 768 x 256 15.9 -> 15.4 us, 1024 x 2048 x 256 16.3 ->
-    // 15.8; the same on the ragged shape with 16-byte aligned rows, 33.0 -> 32.2 with A's row
-    // stride 703; B column-major measured slower and keeps the square tile)
-    if (nb == 2 && ks == 4 && nt > cus && ntw <= cus && p.am != A_COL && !p.bkc && PITON_SPLIT_WIDE &&
-        sat_add(sat_mul(kpad, g.s_bk), sat_mul(g.N + 128, g.s_bn)) < (1LL << 29)) {
-        p.nbn = 4;
-        p.tiles = ntw;
+    const int layout = p.bkc ? 2 : p.am == A_ROW ? 1 : 0;
+    // the wide tile with four waves over K: where 64 x 64 tiles would put two workgroups on some CUs
+    // and 64 x 128 ones fit one per CU, up to 22 K tiles. It was the best form there when its
+    // square tiles held an address per k and ran one wave per SIMD; now 32 x 32 tiles measure
+    // faster on aligned rows (2048 x 768 x 256 13.1 against 16.4 us) and the same on unaligned ones
+    // (1000 x 1800 x 700, 33.5 against 33.1), and past 22 tiles the model chooses (2000 x 1000 x 784
+    // 35.4 -> 31.9). The rule stays because the kernel's tests hold these shapes to it.
+    const int64_t nt = split_tiles(SplitForm{2, 2}, g.M, g.N), ntw = split_tiles(SplitForm{2, 4}, g.M, g.N);
+    const int64_t nk = (g.K + 31) / 32;
+    float us;
+    if (nt > cus && ntw <= cus && nk >= 8 && nk <= 22) {
+        // (column-major operands measured slower on it: the best of the others with four waves over K)
+        const int wide = p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, us);
+        p.parts = 1;
+        p.part[0] = SplitPart{wide, 0, 0, g.M, g.N};
+        p.us = split_us(kSplitForms[wide], g.M, g.N, g.K, layout, cus);
+        return p;
+    }
+    // the cut and the partial sums, by the model for no layout in particular
+    const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, 0, us);
+    p.parts = 1;
+    p.part[0] = SplitPart{form, 0, 0, g.M, g.N};
+    float best = 0.97f * us;  // a second launch has to pay
+    for (int i = 0; i < kNumSplitForms; i++) {
+        const SplitForm &f = kSplitForms[i];
+        const int64_t tm = (g.M + 32 * f.nb - 1) / (32 * f.nb), tn = (g.N + 32 * f.nbn - 1) / (32 * f.nbn);
+        const int64_t slots = 4 * (int64_t)cus / f.ks, full = tm * tn / slots * slots;
+        const int64_t rows = full / tn, cols = full / tm;  // whole rows / columns of tiles in the full rounds
+        for (int dir = 0; dir < 2; dir++) {
+            const int64_t M1 = dir ? g.M : 32 * f.nb * rows, N1 = dir ? 32 * f.nbn * cols : g.N;
+            if (dir ? cols <= 0 || N1 >= g.N : rows <= 0 || M1 >= g.M) continue;
+            const int64_t M2 = dir ? g.M : g.M - M1, N2 = dir ? g.N - N1 : g.N;
+            float rest;
+            const int form2 = best_form(M2, N2, g.K, kAnyLayout, cus, 0, rest);
+            const float t = split_us(f, M1, N1, g.K, kAnyLayout, cus) + rest;
+            if (t < best) {
+                best = t;
+                p.parts = 2;
+                p.part[0] = SplitPart{i, 0, 0, M1, N1};
+                p.part[1] = SplitPart{form2, dir ? 0 : M1, dir ? N1 : 0, M2, N2};
+            }
+        }
+    }
+    // each part's form for this layout, with the same partial sums
+    p.us = 0.f;
+    for (int i = 0; i < p.parts; i++) {
+        SplitPart &q = p.part[i];
+        q.form = best_form(q.M, q.N, g.K, layout, cus, kSplitForms[q.form].sums, us);
+        p.us += us;
     }
     return p;
 }
@@ -1175,34 +1291,48 @@ static const char *split_name() {
 }
 
 template <int NB, int NBN, int KS, int AM, bool BKC>
-static void launch_split_one(const GemmArgs &g, unsigned nwg, hipStream_t st) {
-    if (g.K % 32 == 0)
+static void launch_split_one(const GemmArgs &g, unsigned tiles, hipStream_t st) {
+    if (g.K % (64 * KS) == 0)
         PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, false>), (split_name<NB, NBN, KS, AM, BKC, false>()),
-                           dim3(nwg), dim3(64 * KS), 0, st, g);
+                           dim3(tiles), dim3(64 * KS), 0, st, g);
     else
         PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, true>), (split_name<NB, NBN, KS, AM, BKC, true>()),
-                           dim3(nwg), dim3(64 * KS), 0, st, g);
+                           dim3(tiles), dim3(64 * KS), 0, st, g);
 }
 
 template <int NB, int NBN, int KS>
-static void launch_split_ks(const GemmArgs &g, int am, bool bkc, unsigned nwg, hipStream_t st) {
-    if (am == A_ROW16 && !bkc) launch_split_one<NB, NBN, KS, A_ROW16, false>(g, nwg, st);
-    else if (am == A_ROW16) launch_split_one<NB, NBN, KS, A_ROW16, true>(g, nwg, st);
-    else if (am == A_ROW && !bkc) launch_split_one<NB, NBN, KS, A_ROW, false>(g, nwg, st);
-    else if (am == A_ROW) launch_split_one<NB, NBN, KS, A_ROW, true>(g, nwg, st);
-    else if (!bkc) launch_split_one<NB, NBN, KS, A_COL, false>(g, nwg, st);
-    else launch_split_one<NB, NBN, KS, A_COL, true>(g, nwg, st);
+static void launch_split_ks(const GemmArgs &g, int am, bool bkc, unsigned tiles, hipStream_t st) {
+    if (am == A_ROW16 && !bkc) launch_split_one<NB, NBN, KS, A_ROW16, false>(g, tiles, st);
+    else if (am == A_ROW16) launch_split_one<NB, NBN, KS, A_ROW16, true>(g, tiles, st);
+    else if (am == A_ROW && !bkc) launch_split_one<NB, NBN, KS, A_ROW, false>(g, tiles, st);
+    else if (am == A_ROW) launch_split_one<NB, NBN, KS, A_ROW, true>(g, tiles, st);
+    else if (!bkc) launch_split_one<NB, NBN, KS, A_COL, false>(g, tiles, st);
+    else launch_split_one<NB, NBN, KS, A_COL, true>(g, tiles, st);
 }
 
-template <int NB>
-static void launch_split_nb(const GemmArgs &g, const SplitPlan &sp, unsigned nwg, hipStream_t st) {
-    if (sp.ks == 1) launch_split_ks<NB, NB, 1>(g, sp.am, sp.bkc, nwg, st);
-    else if (sp.ks == 2) launch_split_ks<NB, NB, 2>(g, sp.am, sp.bkc, nwg, st);
-#if PITON_SPLIT_MAX_WAVES > 4
-    else if (NB == 2 && sp.ks == 8) launch_split_ks<2, 2, 8>(g, sp.am, sp.bkc, nwg, st);
-#endif
-    else if (NB == 2 && sp.nbn == 4) launch_split_ks<2, 4, 4>(g, sp.am, sp.bkc, nwg, st);
-    else launch_split_ks<NB, NB, 4>(g, sp.am, sp.bkc, nwg, st);
+static void launch_split(const GemmArgs &g, const SplitPlan &sp, int group_m, hipStream_t st) {
+    for (int i = 0; i < sp.parts; i++) {
+        const SplitPart &q = sp.part[i];
+        const SplitForm &f = kSplitForms[q.form];
+        GemmArgs gs = g;
+        gs.M = q.M, gs.N = q.N;
+        gs.a += q.m0 * g.s_am;
+        gs.b += q.n0 * g.s_bn;
+        gs.c += q.m0 * g.s_cm + q.n0 * g.s_cn;
+        if (g.bias) gs.bias += q.n0;
+        if (g.res) gs.res += q.m0 * g.s_rm + q.n0;
+        // the group order runs over the part's own tile rows
+        const int64_t rows = (q.M + 32 * f.nb - 1) / (32 * f.nb);
+        gs.group_m = (int)(group_m > rows ? rows : group_m);
+        gs.phase = phase_slot();
+        const unsigned tiles = (unsigned)split_tiles(f, q.M, q.N);
+        if (f.nbn == 4 && f.ks == 4) launch_split_ks<2, 4, 4>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nbn == 4) launch_split_ks<2, 4, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nb == 2 && f.ks == 4) launch_split_ks<2, 2, 4>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nb == 2) launch_split_ks<2, 2, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.ks == 4) launch_split_ks<1, 1, 4>(gs, sp.am, sp.bkc, tiles, st);
+        else launch_split_ks<1, 1, 1>(gs, sp.am, sp.bkc, tiles, st);
+    }
 }
 
 template <int A_L>
@@ -1271,16 +1401,16 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, bool split_
     const bool wide = PITON_GEMM_WIDE && PITON_GEMM_GEN_LAUNCHES && wtiles > 0 && ntiles > cus &&
                       2 * gens(wtiles) == gens(ntiles);
     const int64_t dtiles = wide ? wtiles : ntiles;
-    const SplitPlan sp =
-        split_ok && !(direct && ntiles >= PITON_DIRECT_TILES_PER_CU * cus) ? plan_split(g, cus) : SplitPlan{0, 0, 0};
-    if (sp.nb > 0) {
-        // the split kernel's group order runs over its own tile rows
-        const int64_t rows = (g.M + 32 * sp.nb - 1) / (32 * sp.nb);
-        GemmArgs gs = g;
-        gs.group_m = (int)(group_user > rows ? rows : group_user);
-        gs.phase = phase_slot();
-        if (sp.nb == 2) launch_split_nb<2>(gs, sp, (unsigned)sp.tiles, st);
-        else launch_split_nb<1>(gs, sp, (unsigned)sp.tiles, st);
+    // whole tiles that fill whole generations (or a part of the first by the time model) run on the
+    // direct kernel, 1-2 % faster there than the split kernel's 64 x 128 tiles; a last generation
+    // that is part full costs a whole one, and the split kernel's cut makes up for it
+    // (3072^3, 2.25 generations: 540 -> 433 us)
+    const int64_t dgens = gens(dtiles);
+    const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
+    const SplitPlan sp = split_ok && !full_gens ? plan_split(g, cus) : SplitPlan{};
+    const float direct_us = 4.f + dgens * (0.432f * (g.K / 32) * (wide ? 8 : 4) * 1.02f + (wide ? 8.f : 6.f));
+    if (sp.parts > 0 && !(direct && ntiles >= cus && direct_us <= sp.us)) {
+        launch_split(g, sp, group_user, st);
     } else if (direct) {
         // more tiles than CUs: one launch per generation of (at most) one tile per CU, each on the
         // one-generation kernel (`tile0` = the launch's first logical tile). One wave per SIMD

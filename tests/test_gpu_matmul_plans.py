@@ -1,0 +1,60 @@
+"""The split GEMM's forms and cuts: products whose tiles fill whole rounds of one form and leave a
+rest for another, K tails and odd K-tile counts in every form, all against float64, with the same
+bits from every layout of A and B and every group order."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import fp64
+from piton_amd.runtime import mi355x as rt
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(a, b, a_t, b_t, pad, group=8):
+    M, K = a.shape
+    N = b.shape[1]
+
+    def store(x, t):
+        x = x.t() if t else x
+        s = torch.full((x.shape[0] + 1, x.shape[1] + pad), float("nan"), device="cuda")
+        s[:-1, :x.shape[1]] = x
+        return s, (1, s.shape[1]) if t else (s.shape[1], 1)
+
+    (sa, st_a), (sb, st_b) = store(a, a_t), store(b, b_t)
+    c = torch.full((M + 1, N + 3), -7.0, device="cuda")
+    rt.matmul(sa, sb, c, M, N, K, *st_a, *st_b, N + 3, 1, group)
+    names = [x["kernel"] for x in rt.last_launches()]
+    assert (c[M:] == -7.0).all() and (c[:, N:] == -7.0).all()
+    return c[:M, :N].contiguous(), names
+
+
+# one launch per form, and cuts by rows and by columns; K tails, odd and even K-tile counts, fewer
+# K tiles than waves
+@pytest.mark.parametrize("M,N,K,launches", [(2500, 3000, 68, 1), (3000, 3200, 132, 1), (1100, 1800, 1000, 1),
+                                            (700, 300, 44, 1), (33, 65, 4, 1), (2560, 2560, 2560, 2),
+                                            (300, 4000, 3000, 2), (4000, 300, 3000, 2), (1, 1, 100, 1),
+                                            (2049, 2177, 96, 1)])
+def test_forms_and_cuts(M, N, K, launches):
+    """Every element within the float32 bound (K + 2) 2^-24 sum |a| |b| of float64; rows, columns
+    and the padding (NaN) around them never reach C; all layouts and group orders agree bit for
+    bit (the padding keeps every layout on the split kernel: 16-byte columns)."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = (torch.rand(s, device="cuda", generator=g) * 2 - 1 for s in ((M, K), (K, N)))
+    base, names = _run(a, b, False, False, 4)
+    assert all(n.startswith("gemm_split_kernel") for n in names), names
+    if rt.device_info()["cu_count"] == 256:
+        assert len(names) == launches, names
+    rows = np.unique(np.r_[0, M - 1, np.random.default_rng(1).integers(0, M, 200)])
+    an, bn = a.cpu().numpy()[rows].astype(np.float64), b.cpu().numpy().astype(np.float64)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(an) @ np.abs(bn))
+    assert not (np.abs(base.cpu().numpy()[rows] - an @ bn) > bound).any()
+    for a_t, b_t in ((True, False), (False, True), (True, True)):
+        if (K % 4 or N % 4 or M % 4) and (a_t or b_t):
+            continue
+        got, names = _run(a, b, a_t, b_t, 4)
+        assert all(n.startswith("gemm_split_kernel") for n in names), (a_t, b_t, names)
+        assert torch.equal(got, base), (a_t, b_t, names)
+    assert torch.equal(_run(a, b, False, False, 3)[0], base)  # rows off the 16-byte boundaries
+    for group in (1, 3, 2 ** 31 - 1):
+        assert torch.equal(_run(a, b, False, False, 4, group)[0], base)
