@@ -1105,6 +1105,13 @@ __global__ __launch_bounds__(64 * SMWAVES) void gemm_small_m_kernel(GemmArgs g) 
     g.c[mo * g.s_cm + n] = v;
 }
 
+static bool small_m_fast(const GemmArgs &g) {
+    return g.K % (16 * SMWAVES) == 0 && g.s_am % 4 == 0 && aligned16(g.a);
+}
+static dim3 small_m_grid(const GemmArgs &g) {
+    return dim3((unsigned)((g.N + SMN - 1) / SMN), (unsigned)((g.M + 15) / 16));
+}
+
 // the FAST small-M kernel, with the whole K range of a lane group loaded at once where K is
 // 256, 512 or 1024 (the decoder's products: 1024 in one round trip instead of two)
 template <bool LN>
@@ -1161,6 +1168,8 @@ constexpr SplitForm kSplitForms[] = {
 };
 constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
 constexpr int kSplitWide = 3;  // the index of <2, 4, 4>
+constexpr int kDenseChainSums = 4;               // the partial sums mlp3_kernel keeps (mlp.hip)
+constexpr int64_t kDenseChainRows = 1 << 20;     // rows of up to 256 floats within the split kernel's offsets
 
 static int64_t split_tiles(const SplitForm &f, int64_t M, int64_t N) {
     return sat_mul((M + 32 * f.nb - 1) / (32 * f.nb), (N + 32 * f.nbn - 1) / (32 * f.nbn));
@@ -1207,7 +1216,8 @@ struct SplitPlan {
     bool bkc;  // B column-major
     float us;
 };
-static SplitPlan plan_split(const GemmArgs &g, int cus) {
+// sums: 0, or the partial sums every element must have (one launch then, without a cut).
+static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
     SplitPlan p{0, {}, 0, false, 0.f};
     if (g.K <= 0 || g.M <= 0 || g.N <= 0) return p;
     // A with stride 1 along K (16-byte loads where its rows are 16-byte aligned and K % 4 == 0) or
@@ -1246,11 +1256,11 @@ static SplitPlan plan_split(const GemmArgs &g, int cus) {
         return p;
     }
     // the cut and the partial sums, by the model for no layout in particular
-    const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, 0, us);
+    const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, sums, us);
     p.parts = 1;
     p.part[0] = SplitPart{form, 0, 0, g.M, g.N};
     float best = 0.97f * us;  // a second launch has to pay
-    for (int i = 0; i < kNumSplitForms; i++) {
+    for (int i = 0; i < kNumSplitForms && !sums; i++) {
         const SplitForm &f = kSplitForms[i];
         const int64_t tm = (g.M + 32 * f.nb - 1) / (32 * f.nb), tn = (g.N + 32 * f.nbn - 1) / (32 * f.nbn);
         const int64_t slots = 4 * (int64_t)cus / f.ks, full = tm * tn / slots * slots;
@@ -1365,10 +1375,10 @@ static void launch_direct(bool one_gen, bool wide, bool akc, bool bkc, const Gem
     }
 }
 
-// split_ok: shapes that give the direct kernel fewer 128 x 128 tiles than CUs, or that are not
-// whole tiles, take the split kernel when each operand has stride 1 along one axis (its k order differs from the LDS kernel's, so
-// the dense entry, whose bits the fused digits chain reproduces, keeps the LDS kernel)
-static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, bool split_ok) {
+// Whole tiles that fill whole generations take the direct kernel, other shapes the split kernel when
+// each operand has stride 1 along one axis, the rest the LDS kernel. sums: 0, or the partial sums
+// an element must have (plan_split): then the split kernel alone, wherever it applies.
+static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
     if (g.M == 0 || g.N == 0) return PITON_OK;
     const int64_t tiles = sat_mul((g.M + GBM - 1) / GBM, (g.N + GBN - 1) / GBN);
     PITON_REQUIRE(tiles <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "%s: %lld tiles exceed one grid", what, (long long)tiles);
@@ -1407,9 +1417,9 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, bool split_
     // (3072^3, 2.25 generations: 540 -> 433 us)
     const int64_t dgens = gens(dtiles);
     const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
-    const SplitPlan sp = split_ok && !full_gens ? plan_split(g, cus) : SplitPlan{};
+    const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums) : SplitPlan{};
     const float direct_us = 4.f + dgens * (0.432f * (g.K / 32) * (wide ? 8 : 4) * 1.02f + (wide ? 8.f : 6.f));
-    if (sp.parts > 0 && !(direct && ntiles >= cus && direct_us <= sp.us)) {
+    if (sp.parts > 0 && (sums || !(direct && ntiles >= cus && direct_us <= sp.us))) {
         launch_split(g, sp, group_user, st);
     } else if (direct) {
         // more tiles than CUs: one launch per generation of (at most) one tile per CU, each on the
@@ -1453,7 +1463,7 @@ int32_t piton_mi355x_matmul(const float *a, const float *b, float *c, int64_t M,
     if (rc) return rc;
     GemmArgs g{a, b, c, M, N, K, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
                group_size_m, nullptr, 0, nullptr, 0, 0, 0};
-    rc = launch_gemm(g, (hipStream_t)stream, "matmul", true);
+    rc = launch_gemm(g, (hipStream_t)stream, "matmul", 0);
     if (rc == PITON_OK) clear_error();
     return rc;
 }
@@ -1474,7 +1484,25 @@ int32_t piton_mi355x_dense(const float *x, const float *w, const float *bias, fl
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
     GemmArgs g{x, w, y, M, N, K, K, 1, N, 1, N, 1, 1, add_bias ? bias : nullptr, relu ? 1 : 0, nullptr, 0, 0, 0};
-    rc = launch_gemm(g, st, "dense", false);
+    // As the linear entry: 16 waves over K for up to 64 rows, else the split kernel, whose tiles fill
+    // the chip where the LDS kernel's 128 x 128 ones left it idle (64 x 1024 x 1024 92.6 -> 5.3 us,
+    // 2000 x 1000 x 784 75.8 -> 39.4, 4 x 135 x 38 12.4 -> 4.0). Layers that the fused chain takes
+    // too (K even, K and N up to 256) add every element in the order mlp3_kernel does, four partial
+    // sums, whatever their number of rows: in launches of rows that the split kernel's offsets reach
+    const bool chain = K <= 256 && N <= 256 && K % 2 == 0;
+    if (chain) {
+        for (int64_t m = 0; m < M && !rc; m += kDenseChainRows) {
+            g.M = std::min(M - m, kDenseChainRows);
+            g.a = x + m * K;
+            g.c = y + m * N;
+            rc = launch_gemm(g, st, "dense", kDenseChainSums);
+        }
+    } else if (M > 0 && M <= 64 && small_m_fast(g) && (N + SMN - 1) / SMN <= 0x7FFFFFFF) {
+        launch_small_m<false>(g, small_m_grid(g), dim3(64 * SMWAVES), st);
+        rc = check_launch("dense");
+    } else {
+        rc = launch_gemm(g, st, "dense", 0);
+    }
     if (rc) return rc;
     if (argmax_out && M > 0) {
         PITON_REQUIRE((M + 3) / 4 <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "dense: M=%lld too large", (long long)M);
@@ -1504,14 +1532,14 @@ int32_t piton_mi355x_linear(const float *x, int64_t ldx, const float *w, const f
     GemmArgs g{x, w, y, M, N, K, ldx, 1, N, 1, ldy, 1, 1, bias, relu ? 1 : 0, residual, ldr, 0, 0, 0.f};
     if (M > 0 && M <= 64) {
         PITON_REQUIRE((N + SMN - 1) / SMN <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "linear: N=%lld too large", (long long)N);
-        const dim3 grid((unsigned)((N + SMN - 1) / SMN), (unsigned)((M + 15) / 16)), block(64 * SMWAVES);
-        if (K % (16 * SMWAVES) == 0 && ldx % 4 == 0 && aligned16(x))
+        const dim3 grid = small_m_grid(g), block(64 * SMWAVES);
+        if (small_m_fast(g))
             launch_small_m<false>(g, grid, block, (hipStream_t)stream);
         else
             PITON_LAUNCH((gemm_small_m_kernel<false, false>), grid, block, 0, (hipStream_t)stream, g);
         rc = check_launch("linear");
     } else {
-        rc = launch_gemm(g, (hipStream_t)stream, "linear", true);
+        rc = launch_gemm(g, (hipStream_t)stream, "linear", 0);
     }
     if (rc == PITON_OK) clear_error();
     return rc;
@@ -1537,8 +1565,7 @@ int32_t piton_mi355x_linear_ln(const float *x, int64_t ldx, float eps, const flo
     if (rc) return rc;
     if (M == 0) return PITON_OK;
     GemmArgs g{x, w, y, M, N, K, ldx, 1, N, 1, ldy, 1, 1, bias, relu ? 1 : 0, residual, ldr, 0, 0, eps};
-    const dim3 grid((unsigned)((N + SMN - 1) / SMN), (unsigned)((M + 15) / 16)), block(64 * SMWAVES);
-    launch_small_m<true>(g, grid, block, (hipStream_t)stream);
+    launch_small_m<true>(g, small_m_grid(g), dim3(64 * SMWAVES), (hipStream_t)stream);
     rc = check_launch("linear_ln");
     if (rc == PITON_OK) clear_error();
     return rc;

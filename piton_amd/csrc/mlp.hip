@@ -4,12 +4,13 @@
 // The digits networks (64 -> 128 -> 64 -> 10 or 16) take mlp3_rows16_kernel below: 16 rows per
 // workgroup on 16x16x4 MFMAs. Other sizes take mlp3_kernel: a workgroup of four waves takes 32
 // rows through all three layers with the activations in LDS: layer l's 32-column output tiles go
-// to waves round-robin, each computed as one v_mfma_f32_32x32x2_f32 chain over the whole K in
-// ascending k pairs -- the order the dense GEMM uses -- then bias, ReLU (hidden layers) and the
-// fp32 store, so its logits are the three dense launches' logits bit for bit. The A operand (the
-// previous layer's rows) comes from LDS (row pitch 257: conflict-free), the B operand (weights,
-// L2-resident after the first workgroups) from memory, a chunk of 32 k pairs loaded ahead of
-// its MFMAs. The argmax follows numpy's rule (first index of the maximum; a NaN wins), the rule
+// to waves round-robin, each computed by v_mfma_f32_32x32x2_f32 in the order of the split GEMM's
+// forms with four waves over K (K tiles of 32 dealt to four sums, the partial tile first; lane half
+// h supplies k = 16 h + s of a tile at step s; the sums added in order), then bias, ReLU (hidden
+// layers) and the fp32 store, so its logits are the three dense launches' logits bit for bit. The A
+// operand (the previous layer's rows) comes from LDS (row pitch 257: conflict-free), the B operand
+// (weights, L2-resident after the first workgroups) from memory, four K tiles loaded ahead of
+// their MFMAs. The argmax follows numpy's rule (first index of the maximum; a NaN wins), the rule
 // of the dense entry's fused argmax.
 #include "common.h"
 
@@ -21,30 +22,60 @@ constexpr int MLP_ROWS = 32, MLP_PITCH = 257, MLP_MAXK = 256;
 __device__ __forceinline__ void mlp_layer(const float (*in)[MLP_PITCH], int k, const float *w, const float *b, int n,
                                           bool relu, float (*out)[MLP_PITCH]) {
     typedef float f32x16 __attribute__((ext_vector_type(16)));
+    constexpr int SUMS = 4;  // kDenseChainSums
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, half = lane >> 5, l31 = lane & 31;
-    const int ntiles = (n + 31) / 32, steps = k / 2;
+    const int ntiles = (n + 31) / 32, nk = k / 32;
     for (int tile = wave; tile < ntiles; tile += 4) {
         const int col = 32 * tile + l31;
         const bool col_ok = col < n;
-        f32x16 acc;
+        f32x16 sum[SUMS];
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0.f;
-        for (int s0 = 0; s0 < steps; s0 += 32) {
-            float bw[32];
+        for (int u = 0; u < SUMS; u++)
 #pragma unroll
-            for (int u = 0; u < 32; u++) {
-                // an unconditional load from a clamped (valid) address, then the select: a
-                // conditional load becomes a branch whose join waits for it, one load at a time
-                const bool ok = s0 + u < steps && col_ok;
-                const int kk = ok ? 2 * (s0 + u) + half : 0, cc = ok ? col : 0;
-                const float v = w[(int64_t)kk * n + cc];
-                bw[u] = ok ? v : 0.f;
+            for (int r = 0; r < 16; r++) sum[u][r] = 0.f;
+        // whole K tiles need no select: a column past n reads column n - 1 (an output column depends
+        // on its own weight column only, and those past n are not stored), and a tile's rows are a
+        // scalar distance from the lane's offset
+        const uint32_t lane_off = (uint32_t)(16 * half * n + (col_ok ? col : n - 1));
+        auto load = [&](int kt, float (&bw)[16]) {
+#pragma unroll
+            for (int s = 0; s < 16; s++) bw[s] = (w + (int64_t)(32 * kt + s) * n)[lane_off];
+        };
+        auto mul = [&](int kt, const float (&bw)[16], f32x16 &acc) {
+            const float *a = &in[l31][32 * kt + 16 * half];
+#pragma unroll
+            for (int s = 0; s < 16; s++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], bw[s], acc, 0, 0, 0);
+        };
+        if (k % 32 != 0) {
+            // the partial tile: clamped (valid) addresses, then selects: a conditional load becomes a
+            // branch whose join waits for it, one load at a time
+            float aw[16], bw[16];
+#pragma unroll
+            for (int s = 0; s < 16; s++) {
+                const int kk = 32 * nk + 16 * half + s;
+                const bool ok = kk < k;
+                const float av = in[l31][ok ? kk : 0], bv = w[(ok ? kk : 0) * n + (col_ok ? col : n - 1)];
+                aw[s] = ok ? av : 0.f;
+                bw[s] = ok ? bv : 0.f;
             }
 #pragma unroll
-            for (int u = 0; u < 32; u++)
-                if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(in[l31][2 * (s0 + u) + half], bw[u], acc,
-                                                                                0, 0, 0);
+            for (int u = 0; u < SUMS; u++)
+                if (nk % SUMS == u)
+#pragma unroll
+                    for (int s = 0; s < 16; s++)
+                        sum[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(aw[s], bw[s], sum[u], 0, 0, 0);
         }
+        for (int kt = 0; kt < nk; kt += SUMS) {
+            float bw[SUMS][16];
+#pragma unroll
+            for (int u = 0; u < SUMS; u++) load(min(kt + u, nk - 1), bw[u]);
+#pragma unroll
+            for (int u = 0; u < SUMS; u++)
+                if (kt + u < nk) mul(kt + u, bw[u], sum[u]);
+        }
+        f32x16 acc = sum[0];
+#pragma unroll
+        for (int u = 1; u < SUMS; u++) acc += sum[u];
         // accumulator r: row 8*(r/4) + 4*half + r%4, column col
         const float bias = (b && col_ok) ? b[col] : 0.f;
 #pragma unroll
