@@ -1,7 +1,7 @@
 """`@jit`: a Triton-style decorator around a kernel function (piton/jit.py:1-41)."""
 from __future__ import annotations
 
-import inspect
+from .runtime.launcher import Launcher, Parameters
 
 
 def cdiv(a, b):
@@ -24,14 +24,14 @@ class JITFunction:
         self.fn = fn
         self.__name__ = fn.__name__
         self.__doc__ = fn.__doc__
-        self.arg_names = list(inspect.signature(fn).parameters)
+        self.parameters = Parameters(fn)
+        self.arg_names = list(self.parameters.names)
         self._cache = {}
 
     def __call__(self, *args, **kwargs):
         raise RuntimeError("@piton.jit kernels are launched with kernel[grid](...)")
 
     def __getitem__(self, grid):
-        from .runtime.launcher import Launcher
         return Launcher(self, grid)
 
     def __repr__(self):

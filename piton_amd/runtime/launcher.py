@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import inspect
 import os
+import sys
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -29,11 +30,8 @@ _DTYPE_SIG = {np.dtype(np.float32): "*fp32", np.dtype(np.int32): "*i32", np.dtyp
 
 
 def _is_tensor(v) -> bool:
-    try:
-        import torch
-    except ImportError:  # pragma: no cover
-        return False
-    return isinstance(v, torch.Tensor)
+    cls = getattr(sys.modules.get("torch"), "Tensor", None)  # torch not imported: nothing is a tensor
+    return cls is not None and isinstance(v, cls)
 
 
 def _sig_of(value):
@@ -45,7 +43,7 @@ def _sig_of(value):
         return _DTYPE_SIG[value.dtype]
     if _is_tensor(value):
         import torch
-        sig = {torch.float32: "*fp32", torch.int32: "*i32"}.get(value.dtype)
+        sig = "*fp32" if value.dtype == torch.float32 else "*i32" if value.dtype == torch.int32 else None
         if sig is None:
             raise TypeError(f"unsupported tensor dtype {value.dtype} (use float32/int32)")
         return sig
@@ -58,29 +56,66 @@ def _sig_of(value):
     raise TypeError(f"unsupported kernel argument {type(value).__name__}")
 
 
+_ABSENT = object()
+
+
+class Parameters:
+    """A kernel function's parameters, inspected once (inspecting and binding them through
+    `inspect` on every call took 27 us of a matmul launch's host time; `bind` takes 5)."""
+
+    def __init__(self, fn):
+        self.signature = inspect.signature(fn)
+        params = self.signature.parameters.values()
+        self.names = tuple(p.name for p in params)
+        self.name_set = frozenset(self.names)
+        # (name, constexpr?, default)
+        self.params = tuple((p.name, p.annotation is constexpr or
+                             (isinstance(p.annotation, str) and "constexpr" in p.annotation), p.default) for p in params)
+        self.plain = all(p.kind is inspect.Parameter.POSITIONAL_OR_KEYWORD for p in params)
+
+    def arguments(self, args, kwargs):
+        """name -> argument; whatever does not match the parameters raises inspect's TypeError."""
+        if self.plain and len(args) <= len(self.names):
+            bound = dict(zip(self.names, args))
+            n = len(bound)
+            bound.update(kwargs)
+            # no keyword repeats a positional argument, none is unknown
+            if len(bound) == n + len(kwargs) and self.name_set.issuperset(kwargs):
+                return bound
+        return self.signature.bind_partial(*args, **kwargs).arguments
+
+    def bind(self, args, kwargs, do_not_specialize=()):
+        """Split launch arguments into (signature, constants, runtime values), as
+        piton/runtime/launcher.py:42-63 does."""
+        bound = self.arguments(args, kwargs)
+        signature, constants, values = {}, {}, {}
+        for name, is_constexpr, default in self.params:
+            v = bound.get(name, _ABSENT)
+            if v is _ABSENT:
+                if default is inspect.Parameter.empty:
+                    raise TypeError(f"missing kernel argument '{name}'")
+                constants[name] = default.value if isinstance(default, constexpr) else default
+            elif is_constexpr:
+                constants[name] = v
+            elif type(v) is int:
+                if v == 1 and name not in do_not_specialize:
+                    constants[name] = 1
+                else:
+                    signature[name] = "i32"
+                    values[name] = v
+            else:
+                sig = _sig_of(v)
+                if sig == "i32" and v == 1 and name not in do_not_specialize:
+                    constants[name] = 1
+                else:
+                    signature[name] = sig
+                    values[name] = v
+        return signature, constants, values
+
+
 def bind(fn, args, kwargs, do_not_specialize=()):
-    """Split launch arguments into (signature, constants, runtime values), as
-    piton/runtime/launcher.py:42-63 does."""
-    params = list(inspect.signature(fn).parameters.values())
-    bound = inspect.signature(fn).bind_partial(*args, **kwargs)
-    signature, constants, values = {}, {}, {}
-    for p in params:
-        if p.name not in bound.arguments:
-            if p.default is inspect.Parameter.empty:
-                raise TypeError(f"missing kernel argument '{p.name}'")
-            constants[p.name] = p.default.value if isinstance(p.default, constexpr) else p.default
-            continue
-        v = bound.arguments[p.name]
-        ann = p.annotation
-        if ann is constexpr or (isinstance(ann, str) and "constexpr" in ann):
-            constants[p.name] = v
-        elif isinstance(v, (int, np.integer)) and not isinstance(v, bool) and v == 1 \
-                and p.name not in do_not_specialize:
-            constants[p.name] = 1
-        else:
-            signature[p.name] = _sig_of(v)
-            values[p.name] = v
-    return signature, constants, values
+    """Parameters.bind for a function that is not a `JITFunction`'s."""
+    return Parameters(fn).bind(args, kwargs, do_not_specialize)
 
 
 @dataclass
@@ -131,19 +166,35 @@ def plan(jitfn, grid, constants, values):
     """(entry, args) of a launch, with every host-side check done: the grid must be the kernel's
     canonical cover (any other grid would compute a different set of tiles in the reference)."""
     spec = lookup(jitfn)
-    env = _env(grid, constants, values)
+    return spec.entry, _checked_args(jitfn, spec, grid, _env(grid, constants, values))
+
+
+def _checked_args(jitfn, spec, grid, env):
     want = spec.expected_grid(env)
-    if any(w is not None and w != g for w, g in zip(want, env["grid"])):
-        shown = tuple("any" if w is None else w for w in want)
-        raise ValueError(f"{jitfn.__name__}: grid {tuple(grid)} does not cover the kernel's tiles; expected {shown}")
-    for cond, msg in spec.checks:
-        if not cond.py(env):
-            raise ValueError(f"{jitfn.__name__}: {msg}")
-    return spec.entry, spec.args(env)
+    for w, g in zip(want, env["grid"]):
+        if w is not None and w != g:
+            shown = tuple("any" if w is None else w for w in want)
+            raise ValueError(f"{jitfn.__name__}: grid {tuple(grid)} does not cover the kernel's tiles; expected {shown}")
+    msg = spec.failed_check(env)
+    if msg is not None:
+        raise ValueError(f"{jitfn.__name__}: {msg}")
+    return spec.args(env)
 
 
 def _timing() -> bool:
     return os.environ.get("PITON_MI355X_TIMING", "") not in ("", "0")
+
+
+_rt = None
+
+
+def _runtime():
+    """The library binding (imported with the first launch: it loads torch's HIP runtime)."""
+    global _rt
+    if _rt is None:
+        from . import mi355x
+        _rt = mi355x
+    return _rt
 
 
 def run_mi355x(jitfn, grid, signature, constants, values) -> LaunchRecord:
@@ -152,25 +203,26 @@ def run_mi355x(jitfn, grid, signature, constants, values) -> LaunchRecord:
     `jitfn` needs only what the reference's JITFunction carries (piton/jit.py:16-25): `__name__`
     and `arg_names`; `signature`, `constants` and `values` are what the reference's `bind`
     returns for the launch (launcher.py:42-63) and `grid` the resolved grid tuple."""
-    entry, args = plan(jitfn, grid, constants, values)
-    import torch
-
-    from . import mi355x as rt
-    dev = rt.staging_device()
+    spec = lookup(jitfn)
+    env = _env(grid, constants, values)
+    args = _checked_args(jitfn, spec, grid, env)
+    rt = _runtime()
     staged = {}
     for name, v in values.items():
-        if isinstance(v, np.ndarray):
+        if type(v) is not int and isinstance(v, np.ndarray):
+            import torch
             flat = np.ascontiguousarray(v).reshape(-1)
-            staged[name] = torch.from_numpy(flat.view(np.int32) if v.dtype == np.uint32 else flat).to(dev)
-    resolved = [(staged.get(x.name, values.get(x.name)) if isinstance(x, Arr) else x) for x in args]
+            staged[name] = torch.from_numpy(flat.view(np.int32) if v.dtype == np.uint32 else flat).to(rt.staging_device())
+    resolved = [(staged.get(x.name, values.get(x.name)) if type(x) is Arr else x) for x in args]
     timed = _timing()
     if timed:
+        import torch
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record()
-    getattr(rt, entry)(*resolved)
+    getattr(rt, spec.entry)(*resolved)
     if timed:
         e1.record()  # right behind the launch: the host work below is not in the interval
-    stats = {"launches": rt.last_launches(), **lookup(jitfn).work(_env(grid, constants, values))}
+    stats = {"launches": rt.last_launches(), **spec.work(env)}
     if timed:
         e1.synchronize()
         stats["elapsed_us"] = e0.elapsed_time(e1) * 1e3
@@ -179,7 +231,7 @@ def run_mi355x(jitfn, grid, signature, constants, values) -> LaunchRecord:
         for name, t in staged.items():
             v = values[name]
             v[...] = t.cpu().numpy().view(v.dtype).reshape(v.shape)
-    return LaunchRecord(jitfn.__name__, tuple(grid), "piton_mi355x_" + entry, signature, constants, stats)
+    return LaunchRecord(jitfn.__name__, tuple(grid), "piton_mi355x_" + spec.entry, signature, constants, stats)
 
 
 class Launcher:
@@ -189,10 +241,12 @@ class Launcher:
         self.extra_constants = dict(extra_constants or {})
 
     def __call__(self, *args, device: str = "mi355x", num_stages: int = 2, **kwargs):
-        fn = self.jitfn.fn
         for k in ("num_warps", "num_ctas"):
             kwargs.pop(k, None)
-        signature, constants, values = bind(fn, args, kwargs, getattr(self.jitfn, "do_not_specialize", ()))
+        parameters = getattr(self.jitfn, "parameters", None)
+        if not isinstance(parameters, Parameters):
+            parameters = Parameters(self.jitfn.fn)
+        signature, constants, values = parameters.bind(args, kwargs, getattr(self.jitfn, "do_not_specialize", ()))
         constants.update(self.extra_constants)
         grid = self.grid(dict(constants, **values)) if callable(self.grid) else self.grid
         grid = tuple(grid) if isinstance(grid, (tuple, list)) else (grid,)

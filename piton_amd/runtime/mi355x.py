@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
@@ -141,11 +142,23 @@ def device_info() -> dict:
 def last_launches() -> list:
     """The kernel launches of this thread's last entry call: kernel name, grid, block, LDS bytes
     per workgroup, vector registers and spill bytes per lane."""
-    infos = (LaunchInfo * 8)()
-    n = ctypes.c_int32(0)
+    try:
+        infos, n = _notes.buffers
+    except AttributeError:
+        infos, n = _notes.buffers = (LaunchInfo * 8)(), ctypes.c_int32(0)
     _call("piton_mi355x_last_launches", infos, 8, ctypes.byref(n))
-    return [{"kernel": i.kernel.decode(), "grid": tuple(i.grid), "block": tuple(i.block), "lds_bytes": i.lds_bytes,
-             "vgprs": i.vgprs, "scratch_bytes": i.scratch_bytes} for i in infos[:min(n.value, 8)]]
+    # (every launch record reads this; through ctypes' fields one record took 5 us)
+    out = []
+    for i in range(min(n.value, 8)):
+        name, gx, gy, gz, bx, by, bz, lds, vgprs, scratch = _LAUNCH_INFO.unpack_from(infos, i * _LAUNCH_INFO.size)
+        out.append({"kernel": name[:name.index(0)].decode(), "grid": (gx, gy, gz), "block": (bx, by, bz),
+                    "lds_bytes": lds, "vgprs": vgprs, "scratch_bytes": scratch})
+    return out
+
+
+_notes = threading.local()  # a thread's buffers of last_launches
+_LAUNCH_INFO = struct.Struct("96s3I3IIiI")
+assert _LAUNCH_INFO.size == ctypes.sizeof(LaunchInfo)
 
 
 def staging_device() -> str:
@@ -179,7 +192,7 @@ def check_tensor(name: str, t, dtype=torch.float32, max_offset: int | None = Non
         raise TypeError(f"{name}: expected a torch.Tensor, got {type(t).__name__}")
     if t.dtype != dtype:
         raise TypeError(f"{name}: dtype {t.dtype}, expected {dtype}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name}: tensor on {t.device}, expected a ROCm GPU tensor")
     if max_offset is not None and max_offset >= 0 and max_offset >= _avail(t):
         raise ValueError(f"{name}: the kernel addresses element {max_offset} but the storage holds "
@@ -188,7 +201,7 @@ def check_tensor(name: str, t, dtype=torch.float32, max_offset: int | None = Non
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def _span(*pairs) -> int:

@@ -26,7 +26,9 @@ def cdiv(a, b):
 
 
 # -- expressions over the kernel's parameters and the grid -------------------------------------
-# .py(env): the value, env = parameters (values and constants) plus "grid" (three ints);
+# .py: Python source of the value over `env`, parameters (values and constants) plus "grid" (three
+# ints), which a KernelSpec compiles once (evaluating the expressions node by node took 9 us of a
+# matmul launch's host time, the compiled functions take 3);
 # .c(sub): C source, sub(name) = the C expression of parameter `name`.
 
 class Expr:
@@ -40,8 +42,8 @@ class P(Expr):
     def __init__(self, name, conv=int):
         self.name, self.conv = name, conv
 
-    def py(self, env):
-        return self.conv(env[self.name])
+    def py(self):
+        return f"{self.conv.__name__}(env[{self.name!r}])"
 
     def c(self, sub):
         return sub(self.name)
@@ -53,8 +55,8 @@ class Ptr(Expr):
     def __init__(self, name):
         self.name = name
 
-    def py(self, env):
-        return Arr(self.name)
+    def py(self):
+        return f"Arr({self.name!r})"
 
     def c(self, sub):
         return sub(self.name)
@@ -64,8 +66,8 @@ class Null(Expr):
     def __init__(self, ctype):
         self.ctype = ctype
 
-    def py(self, env):
-        return None
+    def py(self):
+        return "None"
 
     def c(self, sub):
         return f"({self.ctype})0"
@@ -75,8 +77,8 @@ class Lit(Expr):
     def __init__(self, v):
         self.v = v
 
-    def py(self, env):
-        return self.v
+    def py(self):
+        return repr(self.v)
 
     def c(self, sub):
         return str(int(self.v))
@@ -86,8 +88,8 @@ class GridDim(Expr):
     def __init__(self, axis):
         self.axis = axis
 
-    def py(self, env):
-        return int(env["grid"][self.axis])
+    def py(self):
+        return f"int(env['grid'][{self.axis}])"
 
     def c(self, sub):
         return f"(long long)g{'xyz'[self.axis]}"
@@ -99,6 +101,9 @@ class _Bin(Expr):
     def __init__(self, a, b):
         self.a, self.b = a, b
 
+    def py(self):
+        return f"({self.a.py()} {self.op} {self.b.py()})"
+
     def c(self, sub):
         return f"({self.a.c(sub)} {self.op} {self.b.c(sub)})"
 
@@ -106,45 +111,36 @@ class _Bin(Expr):
 class Mul(_Bin):
     op = "*"
 
-    def py(self, env):
-        return self.a.py(env) * self.b.py(env)
-
 
 class Mod(_Bin):
     op = "%"
-
-    def py(self, env):
-        return self.a.py(env) % self.b.py(env)
 
 
 class Eq(_Bin):
     op = "=="
 
-    def py(self, env):
-        return self.a.py(env) == self.b.py(env)
-
 
 class Or(_Bin):
     op = "||"
 
-    def py(self, env):
-        return bool(self.a.py(env)) or bool(self.b.py(env))
+    def py(self):
+        return f"(bool({self.a.py()}) or bool({self.b.py()}))"
 
 
 class Not(Expr):
     def __init__(self, a):
         self.a = a
 
-    def py(self, env):
-        return not self.a.py(env)
+    def py(self):
+        return f"(not {self.a.py()})"
 
     def c(self, sub):
         return f"(!{self.a.c(sub)})"
 
 
 class Cdiv(_Bin):
-    def py(self, env):
-        return cdiv(self.a.py(env), self.b.py(env))
+    def py(self):
+        return f"cdiv({self.a.py()}, {self.b.py()})"
 
     def c(self, sub):
         a, b = self.a.c(sub), self.b.c(sub)
@@ -152,8 +148,8 @@ class Cdiv(_Bin):
 
 
 class Min(_Bin):
-    def py(self, env):
-        return min(self.a.py(env), self.b.py(env))
+    def py(self):
+        return f"min({self.a.py()}, {self.b.py()})"
 
     def c(self, sub):
         a, b = self.a.c(sub), self.b.c(sub)
@@ -164,8 +160,8 @@ class Select(Expr):
     def __init__(self, cond, a, b):
         self.cond, self.a, self.b = cond, a, b
 
-    def py(self, env):
-        return self.a.py(env) if self.cond.py(env) else self.b.py(env)
+    def py(self):
+        return f"({self.a.py()} if {self.cond.py()} else {self.b.py()})"
 
     def c(self, sub):
         return f"({self.cond.c(sub)} ? {self.a.c(sub)} : {self.b.c(sub)})"
@@ -181,11 +177,17 @@ class KernelSpec:
     checks: tuple = ()            # (expression that must hold, message)
     work: Callable = field(default=lambda env: {})  # algorithmic flops / bytes of one launch
 
-    def args(self, env):
-        return tuple(e.py(env) for e in self.call)
+    def __post_init__(self):
+        # args(env): the entry's arguments; expected_grid(env): the canonical grid; failed_check(env):
+        # the message of the first check that does not hold, or None
+        self.args = _function(f"({', '.join(e.py() for e in self.call)},)")
+        self.expected_grid = _function(
+            f"({', '.join('None' if g is None else f'int({g.py()})' for g in self.grid)},)")
+        self.failed_check = _function("".join(f"{msg!r} if not {cond.py()} else " for cond, msg in self.checks) + "None")
 
-    def expected_grid(self, env):
-        return tuple(None if g is None else int(g.py(env)) for g in self.grid)
+
+def _function(source):
+    return eval(f"lambda env: {source}", {"Arr": Arr, "cdiv": cdiv})
 
 
 def _mm_work(env):
