@@ -333,6 +333,15 @@ void gemm_f32_kernel(GemmArgs g) {
 #define PITON_GEMM_DIRECT 1
 #endif
 
+// Waits for the values loaded into v here. Left to the compiler, the wait stands at each use: among
+// stores behind branches it then covers the stores too (2048 x 1024 x 256 with bias and ReLU 18.3 us
+// instead of 16.0, 2500 x 3000 x 2000 without either 257 instead of 248).
+template <int N>
+__device__ __forceinline__ void landed(float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
+}
+
 // Whole-tile shapes without LDS: every wave loads its own MFMA operands from memory straight
 // into registers, so there is no LDS staging and no barrier, and the waves of a workgroup run
 // independently. Within a K tile of 32, lane half h supplies k = 16h + s at MFMA step s (the
@@ -500,20 +509,33 @@ void gemm_direct_kernel(GemmArgs g) {
         interleave();
     }
 
-    // accumulator r of a 32x32 block holds row 8*(r/4) + 4*half + r%4, column l31
+    // accumulator r of a 32x32 block holds row 8*(r/4) + 4*half + r%4, column l31. The bias and a
+    // block's residual are requested before the stores that they may alias
+    float bias[WNB] = {};
+    if (g.bias) {
+#pragma unroll
+        for (int nb = 0; nb < WNB; nb++) bias[nb] = g.bias[n0 + wn * 32 * WNB + nb * 32 + l31];
+        landed(bias);
+    }
 #pragma unroll
     for (int mb = 0; mb < DMB; mb++)
 #pragma unroll
         for (int nb = 0; nb < WNB; nb++) {
             const int64_t col = n0 + wn * 32 * WNB + nb * 32 + l31;
-            const float bias = g.bias ? g.bias[col] : 0.f;
+            float res[16] = {};
+            if (g.res) {
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    res[r] = g.res[(m0 + wm * 32 * DMB + mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3)) * g.s_rm + col];
+                landed(res);
+            }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int64_t row = m0 + wm * 32 * DMB + mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
                 float v = acc[mb][nb][r];
-                if (g.bias) v += bias;
+                if (g.bias) v += bias[nb];
                 if (g.relu && v < 0.f) v = 0.f;  // NaN passes, as np.maximum(NaN, 0)
-                if (g.res) v += g.res[row * g.s_rm + col];
+                if (g.res) v += res[r];
                 g.c[row * g.s_cm + col * g.s_cn] = v;
             }
         }
@@ -841,25 +863,65 @@ void gemm_split_kernel(GemmArgs g) {
     }
 
     PITON_PHASE(2);
-    // accumulator r of a 32x32 block holds row 8*(r/4) + 4*half + r%4, column l31
-    auto store = [&](int i, int j, int r, int ln, float v) {
-        const int64_t row = m0 + i * 32 + 8 * (r >> 2) + 4 * (ln >> 5) + (r & 3);
-        const int64_t col = n0 + j * 32 + (ln & 31);
-        if (row >= g.M || col >= g.N) return;
-        if (g.bias) v += g.bias[col];
+    // accumulator r of a 32x32 block holds row 8*(r/4) + 4*half + r%4, column l31. The bias and the
+    // residual of a group are requested before its first store: between the stores, which they may
+    // alias for all the compiler knows, each was a memory round trip
+    auto row_of = [&](int i, int r) { return m0 + i * 32 + 8 * (r >> 2) + 4 * half + (r & 3); };
+    auto bias_of = [&](int j) { return g.bias[min(n0 + j * 32 + l31, g.N - 1)]; };
+    auto res_of = [&](int i, int j, int r) {  // (rows and columns past the edge: the last one's)
+        return g.res[min(row_of(i, r), g.M - 1) * g.s_rm + min(n0 + j * 32 + l31, g.N - 1)];
+    };
+    auto store = [&](int i, int j, int r, float v, float bias, float res, auto whole) {
+        const int64_t row = row_of(i, r), col = n0 + j * 32 + l31;
+        if (!decltype(whole)::value && (row >= g.M || col >= g.N)) return;
+        if (g.bias) v += bias;
         if (g.relu && v < 0.f) v = 0.f;  // NaN passes, as np.maximum(NaN, 0)
-        if (g.res) v += g.res[row * g.s_rm + col];
+        if (g.res) v += res;
         g.c[row * g.s_cm + col * g.s_cn] = v;
     };
+    // tiles without an edge store without a branch per element (1024^3 22.4 -> 21.9 us, 2500 x 3000 x
+    // 2000 247 -> 246, 3072^3 464 -> 458)
+    const bool whole_tile = m0 + TB <= g.M && n0 + TBN <= g.N;
     if constexpr (KS == 1) {
+        float bias[NBN] = {};
+        if (g.bias)
+#pragma unroll
+            for (int j = 0; j < NBN; j++) bias[j] = bias_of(j);
+        landed(bias);
 #pragma unroll
         for (int i = 0; i < NB; i++)
 #pragma unroll
-            for (int j = 0; j < NBN; j++)
+            for (int j = 0; j < NBN; j++) {
+                float res[16] = {};
+                if (g.res)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    store(i, j, r, lane, NSUM == 1 ? acc[0][i][j][r] : acc[0][i][j][r] + acc[NSUM - 1][i][j][r]);
+                    for (int r = 0; r < 16; r++) res[r] = res_of(i, j, r);
+                landed(res);
+                auto put = [&](auto whole) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        store(i, j, r, NSUM == 1 ? acc[0][i][j][r] : acc[0][i][j][r] + acc[NSUM - 1][i][j][r], bias[j],
+                              res[r], whole);
+                };
+                if (whole_tile) put(std::true_type());
+                else put(std::false_type());
+            }
     } else {
+        // wave w finishes the groups w, w + KS, ... of four accumulators (group x: block x / 4,
+        // accumulators 4 (x % 4) .. + 3)
+        constexpr int GPW = NACC / 4 / KS;  // groups per wave
+        float bias[GPW] = {}, res[GPW][4] = {};
+        if (g.bias)
+#pragma unroll
+            for (int u = 0; u < GPW; u++) bias[u] = bias_of(((wave + KS * u) >> 2) % NBN);
+        if (g.res)
+#pragma unroll
+            for (int u = 0; u < GPW; u++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int x = wave + KS * u;
+                    res[u][e] = res_of((x >> 2) / NBN, (x >> 2) % NBN, 4 * (x & 3) + e);
+                }
 #pragma unroll
         for (int i = 0; i < NB; i++)
 #pragma unroll
@@ -875,23 +937,29 @@ void gemm_split_kernel(GemmArgs g) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         __builtin_amdgcn_sched_barrier(0);
-        // wave w finishes the groups w, w + KS, ... of four accumulators, every partial read
-        // first; the partials add in wave order
-        constexpr int GPW = NACC / 4 / KS;  // groups per wave
+        // every partial read first; the partials add in wave order
         f32x4 part[GPW][KS];
 #pragma unroll
         for (int u = 0; u < GPW; u++)
 #pragma unroll
             for (int w = 0; w < KS; w++) part[u][w] = red[w][wave + KS * u][lane];
+        landed(bias);
 #pragma unroll
-        for (int u = 0; u < GPW; u++) {
-            const int x = wave + KS * u;  // group: block x / 4, accumulators 4 (x % 4) .. + 3
-            f32x4 v = part[u][0];
+        for (int u = 0; u < GPW; u++) landed(res[u]);
+        auto put = [&](auto whole) {
 #pragma unroll
-            for (int w = 1; w < KS; w++) v += part[u][w];
+            for (int u = 0; u < GPW; u++) {
+                const int x = wave + KS * u;
+                f32x4 v = part[u][0];
 #pragma unroll
-            for (int e = 0; e < 4; e++) store((x >> 2) / NBN, (x >> 2) % NBN, 4 * (x & 3) + e, lane, v[e]);
-        }
+                for (int w = 1; w < KS; w++) v += part[u][w];
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    store((x >> 2) / NBN, (x >> 2) % NBN, 4 * (x & 3) + e, v[e], bias[u], res[u][e], whole);
+            }
+        };
+        if (whole_tile) put(std::true_type());
+        else put(std::false_type());
     }
     PITON_PHASE(3);
     PITON_PHASE_END(kPhaseGemmSplit, g.phase);
@@ -1168,6 +1236,9 @@ constexpr SplitForm kSplitForms[] = {
 };
 constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
 constexpr int kSplitWide = 3;  // the index of <2, 4, 4>
+// tile rows per group of the entries that have no GROUP_SIZE_M: an XCD's tiles share B's columns
+// and A's rows in its L2 (2000 x 1000 x 784 36.5 us with groups of one row, 34.1 with 4 to 16)
+constexpr int kGroupRows = 8;
 constexpr int kDenseChainSums = 4;               // the partial sums mlp3_kernel keeps (mlp.hip)
 constexpr int64_t kDenseChainRows = 1 << 20;     // rows of up to 256 floats within the split kernel's offsets
 
@@ -1217,7 +1288,7 @@ struct SplitPlan {
     float us;
 };
 // sums: 0, or the partial sums every element must have (one launch then, without a cut).
-static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
+static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule) {
     SplitPlan p{0, {}, 0, false, 0.f};
     if (g.K <= 0 || g.M <= 0 || g.N <= 0) return p;
     // A with stride 1 along K (16-byte loads where its rows are 16-byte aligned and K % 4 == 0) or
@@ -1243,13 +1314,14 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
     // square tiles held an address per k and ran one wave per SIMD; now 32 x 32 tiles measure
     // faster on aligned rows (2048 x 768 x 256 13.1 against 16.4 us) and the same on unaligned ones
     // (1000 x 1800 x 700, 33.5 against 33.1), and past 22 tiles the model chooses (2000 x 1000 x 784
-    // 35.4 -> 31.9). The rule stays because the kernel's tests hold these shapes to it.
+    // 35.4 -> 31.9). The rule stays for the matmul entry (wide_rule), whose tests hold these shapes
+    // to it.
     const int64_t nt = split_tiles(SplitForm{2, 2}, g.M, g.N), ntw = split_tiles(SplitForm{2, 4}, g.M, g.N);
     const int64_t nk = (g.K + 31) / 32;
     float us;
     if (nt > cus && ntw <= cus && nk >= 8 && nk <= 22) {
         // (column-major operands measured slower on it: the best of the others with four waves over K)
-        const int wide = p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, us);
+        const int wide = wide_rule && p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, us);
         p.parts = 1;
         p.part[0] = SplitPart{wide, 0, 0, g.M, g.N};
         p.us = split_us(kSplitForms[wide], g.M, g.N, g.K, layout, cus);
@@ -1378,7 +1450,7 @@ static void launch_direct(bool one_gen, bool wide, bool akc, bool bkc, const Gem
 // Whole tiles that fill whole generations take the direct kernel, other shapes the split kernel when
 // each operand has stride 1 along one axis, the rest the LDS kernel. sums: 0, or the partial sums
 // an element must have (plan_split): then the split kernel alone, wherever it applies.
-static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
+static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums, bool wide_rule) {
     if (g.M == 0 || g.N == 0) return PITON_OK;
     const int64_t tiles = sat_mul((g.M + GBM - 1) / GBM, (g.N + GBN - 1) / GBN);
     PITON_REQUIRE(tiles <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "%s: %lld tiles exceed one grid", what, (long long)tiles);
@@ -1417,7 +1489,7 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
     // (3072^3, 2.25 generations: 540 -> 433 us)
     const int64_t dgens = gens(dtiles);
     const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
-    const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums) : SplitPlan{};
+    const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums, wide_rule) : SplitPlan{};
     const float direct_us = 4.f + dgens * (0.432f * (g.K / 32) * (wide ? 8 : 4) * 1.02f + (wide ? 8.f : 6.f));
     if (sp.parts > 0 && (sums || !(direct && ntiles >= cus && direct_us <= sp.us))) {
         launch_split(g, sp, group_user, st);
@@ -1463,7 +1535,7 @@ int32_t piton_mi355x_matmul(const float *a, const float *b, float *c, int64_t M,
     if (rc) return rc;
     GemmArgs g{a, b, c, M, N, K, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
                group_size_m, nullptr, 0, nullptr, 0, 0, 0};
-    rc = launch_gemm(g, (hipStream_t)stream, "matmul", 0);
+    rc = launch_gemm(g, (hipStream_t)stream, "matmul", 0, true);
     if (rc == PITON_OK) clear_error();
     return rc;
 }
@@ -1483,7 +1555,7 @@ int32_t piton_mi355x_dense(const float *x, const float *w, const float *bias, fl
     int rc = require_device();
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    GemmArgs g{x, w, y, M, N, K, K, 1, N, 1, N, 1, 1, add_bias ? bias : nullptr, relu ? 1 : 0, nullptr, 0, 0, 0};
+    GemmArgs g{x, w, y, M, N, K, K, 1, N, 1, N, 1, kGroupRows, add_bias ? bias : nullptr, relu ? 1 : 0, nullptr, 0, 0, 0};
     // As the linear entry: 16 waves over K for up to 64 rows, else the split kernel, whose tiles fill
     // the chip where the LDS kernel's 128 x 128 ones left it idle (64 x 1024 x 1024 92.6 -> 5.3 us,
     // 2000 x 1000 x 784 75.8 -> 39.4, 4 x 135 x 38 12.4 -> 4.0). Layers that the fused chain takes
@@ -1495,13 +1567,13 @@ int32_t piton_mi355x_dense(const float *x, const float *w, const float *bias, fl
             g.M = std::min(M - m, kDenseChainRows);
             g.a = x + m * K;
             g.c = y + m * N;
-            rc = launch_gemm(g, st, "dense", kDenseChainSums);
+            rc = launch_gemm(g, st, "dense", kDenseChainSums, false);
         }
     } else if (M > 0 && M <= 64 && small_m_fast(g) && (N + SMN - 1) / SMN <= 0x7FFFFFFF) {
         launch_small_m<false>(g, small_m_grid(g), dim3(64 * SMWAVES), st);
         rc = check_launch("dense");
     } else {
-        rc = launch_gemm(g, st, "dense", 0);
+        rc = launch_gemm(g, st, "dense", 0, false);
     }
     if (rc) return rc;
     if (argmax_out && M > 0) {
@@ -1529,7 +1601,7 @@ int32_t piton_mi355x_linear(const float *x, int64_t ldx, const float *w, const f
                   "linear: pointers must be 4-byte aligned");
     int rc = require_device();
     if (rc) return rc;
-    GemmArgs g{x, w, y, M, N, K, ldx, 1, N, 1, ldy, 1, 1, bias, relu ? 1 : 0, residual, ldr, 0, 0, 0.f};
+    GemmArgs g{x, w, y, M, N, K, ldx, 1, N, 1, ldy, 1, kGroupRows, bias, relu ? 1 : 0, residual, ldr, 0, 0, 0.f};
     if (M > 0 && M <= 64) {
         PITON_REQUIRE((N + SMN - 1) / SMN <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "linear: N=%lld too large", (long long)N);
         const dim3 grid = small_m_grid(g), block(64 * SMWAVES);
@@ -1539,7 +1611,7 @@ int32_t piton_mi355x_linear(const float *x, int64_t ldx, const float *w, const f
             PITON_LAUNCH((gemm_small_m_kernel<false, false>), grid, block, 0, (hipStream_t)stream, g);
         rc = check_launch("linear");
     } else {
-        rc = launch_gemm(g, (hipStream_t)stream, "linear", 0);
+        rc = launch_gemm(g, (hipStream_t)stream, "linear", 0, false);
     }
     if (rc == PITON_OK) clear_error();
     return rc;

@@ -56,3 +56,22 @@ def test_fused_chain_adds_as_the_dense_launches(M, sizes):
         assert [l["kernel"].startswith("gemm_split_kernel") for l in rt.last_launches()] == [True]
         h = y
     assert torch.equal(logits, h)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 33, 40), (2048, 768, 256), (700, 1000, 100), (2500, 3000, 68),
+                                   (4000, 300, 2000), (300, 4000, 3000), (4096, 4096, 64)])
+def test_linear_residual_in_place(M, N, K):
+    """bias, ReLU and a residual that is the output itself, rows N + 5 apart, in the split kernel's
+    forms (ragged tiles, one and four waves over K, cuts by rows and by columns) and the direct
+    kernel: within (K + 4) 2^-24 (sum |x| |w| + |b| + |r|) of float64, the padding untouched."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    rand = lambda *s: torch.rand(s, device="cuda", generator=g) * 2 - 1  # noqa: E731
+    x, w, b, y = rand(M, K), rand(K, N), rand(N), rand(M, N + 5)
+    y0 = y.clone()
+    rt.linear(x, K, w, b, y, N + 5, y, N + 5, M, N, K, relu=True)
+    assert torch.equal(y[:, N:], y0[:, N:])
+    rows = torch.from_numpy(np.unique(np.r_[0, M - 1, np.random.default_rng(1).integers(0, M, 200)])).cuda()
+    xd, wd, bd, rd = x[rows].double(), w.double(), b.double(), y0[rows, :N].double()
+    ref = torch.relu(xd @ wd + bd) + rd
+    bound = (K + 4) * 2.0 ** -24 * (xd.abs() @ wd.abs() + bd.abs() + rd.abs())
+    assert not ((y[rows, :N].double() - ref).abs() > bound).any()
