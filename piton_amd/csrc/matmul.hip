@@ -664,15 +664,19 @@ void gemm_split_kernel(GemmArgs g) {
     };
     // PIN keeps the loads in source order with scheduling barriers (A first, then B step by step).
     auto load_tile = [&](int kt, Ops &o, auto pin, auto tail) {
-        constexpr bool T = decltype(tail)::value;
+        constexpr int STEPS = decltype(tail)::value;  // of the partial tile; 0: a whole one
+        constexpr bool T = STEPS > 0;
         const auto ra = rsrc(a_al, a_bound, sak4, kt, nk + T);
         const auto rb = rsrc(g.b, b_bound, sbk4, kt, nk + T);
+        // the offsets hold k = 16 h; the partial tile's start at k = STEPS h
+        const uint32_t back = T ? (uint32_t)(half * (16 - STEPS)) : 0u;
         auto pinned = [&]() {
             if constexpr (decltype(pin)::value) __builtin_amdgcn_sched_barrier(0);
         };
         // k = s of block i: per-lane offsets per k, or per block with the k in the scalar offset
         auto load_k = [&](auto r, const auto &per_k, const auto &per_block, uint32_t step4, int s, int i) {
-            const int off = (int)(KSOFF ? per_block[i] + (T ? s * step4 : 0u) : per_k[s] + 128 * i);
+            const uint32_t start = KSOFF ? per_block[i] - back * step4 : per_k[s] - back * step4;
+            const int off = (int)(start + (KSOFF ? (T ? s * step4 : 0u) : 128u * i));
             return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, KSOFF && !T ? (int)(s * step4) : 0, 0));
         };
 #pragma unroll
@@ -688,7 +692,7 @@ void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
                 for (int q = 0; q < (AVEC ? 4 : 5); q++) {
                     const f32x4 v =
-                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va[i] + 16 * q), 0, 0));
+                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(va[i] - 4 * back + 16 * q), 0, 0));
 #pragma unroll
                     for (int e = 0; e < 4; e++) o.a[i][4 * q + e] = v[e];
                     pinned();
@@ -701,7 +705,7 @@ void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const f32x4 v =
-                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(vb[j] + 16 * q), 0, 0));
+                        __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(vb[j] - 4 * back + 16 * q), 0, 0));
 #pragma unroll
                     for (int e = 0; e < 4; e++) o.b[j][4 * q + e] = v[e];
                     pinned();
@@ -716,7 +720,8 @@ void gemm_split_kernel(GemmArgs g) {
                 }
         }
     };
-    auto load = [&](int kt, Ops &o, auto pin) { load_tile(kt, o, pin, std::false_type()); };
+    using Whole = std::integral_constant<int, 0>;
+    auto load = [&](int kt, Ops &o, auto pin) { load_tile(kt, o, pin, Whole()); };
     using Pin = std::true_type;
     using Free = std::false_type;
     // 64 x 128 and 32 x 32 tiles with one wave over K add even and odd K tiles apart (the registers
@@ -754,11 +759,12 @@ void gemm_split_kernel(GemmArgs g) {
             }
         }
     };
-    // MASKED (the K tail): values with k >= K, which the operands along K may hold from the padding
+    // MASKED (the K tail, `tail` steps of it): values with k >= K, which the operands along K may hold from the padding
     // or the next row or column, are zeros
-    auto mul = [&](const Ops &o, f32x16 (&acc)[NB][NBN], int kt, auto masked) {
-        constexpr bool MASKED = decltype(masked)::value;
-        const int rem = (int)(g.K - (int64_t)kt * 32) - 16 * half;  // this lane's k below K in the tile
+    auto mul = [&](const Ops &o, f32x16 (&acc)[NB][NBN], auto tail) {
+        constexpr bool MASKED = decltype(tail)::value > 0;
+        constexpr int STEPS = MASKED ? decltype(tail)::value : 16;
+        const int rem = (int)(g.K % 32) - STEPS * half;  // MASKED: this lane's k below K in the tile
         float av[NB][16];
 #pragma unroll
         for (int i = 0; i < NB; i++) {
@@ -768,7 +774,7 @@ void gemm_split_kernel(GemmArgs g) {
                 for (int s = 0; s < 16; s++) av[i][s] = s < rem ? av[i][s] : 0.f;
         }
 #pragma unroll
-        for (int s = 0; s < 16; s++)
+        for (int s = 0; s < STEPS; s++)
 #pragma unroll
             for (int j = 0; j < NBN; j++) {
                 const float bv = !(MASKED && BKC) || s < rem ? o.b[j][s] : 0.f;
@@ -836,12 +842,19 @@ void gemm_split_kernel(GemmArgs g) {
     int kt = wave;
     if constexpr (TAIL) {
         if (wave == nk % KS && g.K % 32 != 0) {
-            load_tile(nk, o1, Free(), std::true_type());
-            mul(o1, acc[0], nk, std::true_type());
+            // up to 16 values: 8 to each lane half (k = 8 h + s at step s), half the products (2000 x
+            // 1000 x 784 34.5 -> 32.1 us); apart, since a step count known only at run time made the
+            // longer tails slower (1000 x 1800 x 700 31.5 -> 33.5)
+            auto part = [&](auto steps) {
+                load_tile(nk, o1, Free(), steps);
+                mul(o1, acc[0], steps);
+            };
+            if (g.K % 32 <= 16) part(std::integral_constant<int, 8>());
+            else part(std::integral_constant<int, 16>());
         }
         if (nk > wave && ((nk - wave + KS - 1) / KS) % 2) {
             load(kt + KS, o1, Free());
-            mul(o0, acc[NSUM - 1], kt, std::false_type());
+            mul(o0, acc[NSUM - 1], Whole());
             o0 = o1;
             kt += KS;
             if constexpr (PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // as after the prologue's
@@ -851,13 +864,13 @@ void gemm_split_kernel(GemmArgs g) {
         if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         __builtin_amdgcn_sched_barrier(0);
         load(kt + KS, o1, Free());
-        mul(o0, acc[0], kt, std::false_type());
+        mul(o0, acc[0], Whole());
         interleave();
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
         __builtin_amdgcn_sched_barrier(0);
         load(kt + 2 * KS, o0, Free());
-        mul(o1, acc[NSUM - 1], kt + KS, std::false_type());
+        mul(o1, acc[NSUM - 1], Whole());
         interleave();
         __builtin_amdgcn_sched_barrier(0);
     }

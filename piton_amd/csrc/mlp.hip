@@ -6,7 +6,7 @@
 // rows through all three layers with the activations in LDS: layer l's 32-column output tiles go
 // to waves round-robin, each computed by v_mfma_f32_32x32x2_f32 in the order of the split GEMM's
 // forms with four waves over K (K tiles of 32 dealt to four sums, the partial tile first; lane half
-// h supplies k = 16 h + s of a tile at step s; the sums added in order), then bias, ReLU (hidden
+// h supplies k = 16 h + s of a tile at step s, of a partial one its half; the sums added in order), then bias, ReLU (hidden
 // layers) and the fp32 store, so its logits are the three dense launches' logits bit for bit. The A
 // operand (the previous layer's rows) comes from LDS (row pitch 257: conflict-free), the B operand
 // (weights, L2-resident after the first workgroups) from memory, four K tiles loaded ahead of
@@ -50,10 +50,11 @@ __device__ __forceinline__ void mlp_layer(const float (*in)[MLP_PITCH], int k, c
             // the partial tile: clamped (valid) addresses, then selects: a conditional load becomes a
             // branch whose join waits for it, one load at a time
             float aw[16], bw[16];
+            const int steps = k % 32 <= 16 ? 8 : 16;  // as the split kernel deals a partial tile
 #pragma unroll
             for (int s = 0; s < 16; s++) {
-                const int kk = 32 * nk + 16 * half + s;
-                const bool ok = kk < k;
+                const int kk = 32 * nk + steps * half + s;
+                const bool ok = kk < k && s < steps;
                 const float av = in[l31][ok ? kk : 0], bv = w[(ok ? kk : 0) * n + (col_ok ? col : n - 1)];
                 aw[s] = ok ? av : 0.f;
                 bw[s] = ok ? bv : 0.f;

@@ -58,3 +58,17 @@ def test_forms_and_cuts(M, N, K, launches):
     assert torch.equal(_run(a, b, False, False, 3)[0], base)  # rows off the 16-byte boundaries
     for group in (1, 3, 2 ** 31 - 1):
         assert torch.equal(_run(a, b, False, False, 4, group)[0], base)
+
+
+@pytest.mark.parametrize("M,N,tiles", [(96, 160, 1), (96, 160, 5), (2049, 2177, 2), (600, 1100, 9)])
+def test_every_k_tail(M, N, tiles):
+    """All 31 lengths of the partial K tile (up to 16 values, or more, to the two lane halves), with NaN
+    after A's and B's rows: dyadic inputs, every sum exact, so float64's bits."""
+    g = torch.Generator(device="cuda").manual_seed(M + tiles)
+    for rem in range(1, 32):
+        K = 32 * tiles + rem
+        a, b = (torch.randint(-4, 5, s, device="cuda", generator=g).float() / 4 for s in ((M, K), (K, N)))
+        want = (a.double() @ b.double()).float()
+        for a_t, b_t, pad in ((False, False, 4), (False, False, 3), (True, False, 4), (False, True, 4 - K % 4)):
+            got, names = _run(a, b, a_t, b_t, pad)
+            assert torch.equal(got, want), (K, a_t, b_t, names)
