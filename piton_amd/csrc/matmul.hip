@@ -1571,7 +1571,7 @@ int32_t piton_mi355x_dense(const float *x, const float *w, const float *bias, fl
     GemmArgs g{x, w, y, M, N, K, K, 1, N, 1, N, 1, kGroupRows, add_bias ? bias : nullptr, relu ? 1 : 0, nullptr, 0, 0, 0};
     // As the linear entry: 16 waves over K for up to 64 rows, else the split kernel, whose tiles fill
     // the chip where the LDS kernel's 128 x 128 ones left it idle (64 x 1024 x 1024 92.6 -> 5.3 us,
-    // 2000 x 1000 x 784 75.8 -> 39.4, 4 x 135 x 38 12.4 -> 4.0). Layers that the fused chain takes
+    // 2000 x 1000 x 784 75.8 -> 32.0, 4 x 135 x 38 12.4 -> 4.0). Layers that the fused chain takes
     // too (K even, K and N up to 256) add every element in the order mlp3_kernel does, four partial
     // sums, whatever their number of rows: in launches of rows that the split kernel's offsets reach
     const bool chain = K <= 256 && N <= 256 && K % 2 == 0;
