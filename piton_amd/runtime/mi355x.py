@@ -364,7 +364,6 @@ def attn_decode(q, k, v, out, sm_scale, s_qb, s_qh, s_kb, s_kh, s_kn, s_vb, s_vh
         _call("piton_mi355x_attn_decode_split", *args, _ptr(ws), ws.numel(), _stream())
 
 
-
 def _decode_workspace(n_keys, batch, heads, head_dim):
     """The split decode attention's workspace, or None where the call does not split (or the
     device has no memory left for it: the unsplit kernel needs none)."""
@@ -373,7 +372,8 @@ def _decode_workspace(n_keys, batch, heads, head_dim):
     if n.value == 0:
         return None
     try:
-        return torch.empty(n.value, device="cuda")
+        # (float32 whatever torch's default dtype is: n counts the kernels' floats)
+        return torch.empty(n.value, dtype=torch.float32, device="cuda")
     except torch.OutOfMemoryError:
         return None
 

@@ -196,6 +196,28 @@ def test_tensor_checks():
     assert mi355x._span((4, 10), (3, 1)) == 32 and mi355x._span((0, 5)) == -1
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float64])
+def test_decode_workspace_is_float32_under_any_default_dtype(monkeypatch, dtype):
+    """The split decode attention's workspace holds 4-byte floats, as many as the library asks for,
+    whatever torch's default dtype is (half the bytes would put the kernels' writes past its end)."""
+    floats = 2 * 3 * 5 * 66
+    made, empty = [], torch.empty
+
+    def call(name, *args):
+        assert name == "piton_mi355x_attn_decode_workspace"
+        args[-1]._obj.value = floats
+
+    monkeypatch.setattr(mi355x, "_call", call)
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: made.append(empty(*a, **{**k, "device": "cpu"})) or made[-1])
+    default = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        ws = mi355x._decode_workspace(1200, 2, 3, 64)
+    finally:
+        torch.set_default_dtype(default)
+    assert ws is made[0] and ws.dtype == torch.float32 and ws.numel() * ws.element_size() == 4 * floats
+
+
 # -- the reference-side hunks (INTEGRATION.md) driven on any host ------------------------------------
 
 @pytest.fixture
