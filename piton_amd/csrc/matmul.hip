@@ -571,8 +571,11 @@ void gemm_direct_kernel(GemmArgs g) {
 #define PITON_GEMM_GEN_LAUNCHES 1
 #endif
 enum SplitA { A_ROW16 = 0, A_ROW = 1, A_COL = 2 };
-template <int NB, int NBN, int KS, int AM, bool BKC, bool TAIL>
-__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(1, KS == 1 && NBN == 4 ? 1 : 8)))
+// NSUM: the interleaved partial sums that a wave keeps (its K tiles in turn; added in order at the
+// end). SplitForm::sums is their number over all waves.
+constexpr int loop_k(int ks, int nsum) { return nsum == 4 ? 128 : 64 * ks; }  // the K of a loop pass
+template <int NB, int NBN, int KS, int AM, bool BKC, bool TAIL, int NSUM>
+__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(NSUM == 4 ? 3 : 1, KS == 1 && NBN == 4 ? 1 : 8)))
 void gemm_split_kernel(GemmArgs g) {
     constexpr bool AVEC = AM == A_ROW16;
     constexpr int TB = 32 * NB, TBN = 32 * NBN;  // tile rows and columns
@@ -724,10 +727,11 @@ void gemm_split_kernel(GemmArgs g) {
     auto load = [&](int kt, Ops &o, auto pin) { load_tile(kt, o, pin, Whole()); };
     using Pin = std::true_type;
     using Free = std::false_type;
-    // 64 x 128 and 32 x 32 tiles with one wave over K add even and odd K tiles apart (the registers
-    // are there), so that their sums are no longer chains than two waves over K have: 2500 x 3000 x
-    // 2000 is off float64 by 5.7e-7 so and 8.0e-7 with one chain, at the same speed
-    constexpr int NSUM = KS == 1 && NBN != 2 ? 2 : 1;
+    // 64 x 128 and 32 x 32 tiles with one wave over K deal its K tiles to two sums or four (the
+    // registers are there), so that they are no longer chains than two or four waves over K have: 2500
+    // x 3000 x 2000 is off float64 by 5.7e-7 so and 8.0e-7 with one chain, at the same speed. Four
+    // sums are the bits of four waves
+    static_assert(NSUM == 1 || (KS == 1 && NBN != 2), "several sums: one wave over K");
     f32x16 acc[NSUM][NB][NBN];
 #pragma unroll
     for (int u = 0; u < NSUM; u++)
@@ -837,8 +841,10 @@ void gemm_split_kernel(GemmArgs g) {
     // TAIL, before the loop, which takes pairs of whole tiles: the partial tile, masked (masks inside
     // the loop, a compare and a select per 16-byte chunk and tile, held 2500 x 3000 x 2000 to 0.72 of
     // the matrix rate), and the first tile of a wave with an odd count (a zero tile padded the pair).
-    // The kernel without them is kept for K a multiple of 64 KS: the loop behind them measured 1024^3
+    // The kernel without them is kept for K a multiple of the loop's pass: the loop behind them measured 1024^3
     // at 22.5 us against 21.5.
+    // NSUM == 4: acc[u] takes the K tiles kt with (kt - rot) % 4 == u, acc[0] the partial tile
+    const int rot = NSUM == 4 && TAIL ? nk % 4 : 0;
     int kt = wave;
     if constexpr (TAIL) {
         if (wave == nk % KS && g.K % 32 != 0) {
@@ -852,27 +858,64 @@ void gemm_split_kernel(GemmArgs g) {
             if (g.K % 32 <= 16) part(std::integral_constant<int, 8>());
             else part(std::integral_constant<int, 16>());
         }
-        if (nk > wave && ((nk - wave + KS - 1) / KS) % 2) {
-            load(kt + KS, o1, Free());
-            mul(o0, acc[NSUM - 1], Whole());
-            o0 = o1;
-            kt += KS;
-            if constexpr (PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // as after the prologue's
+        if constexpr (NSUM < 4) {
+            if (nk > wave && ((nk - wave + KS - 1) / KS) % 2) {
+                load(kt + KS, o1, Free());
+                mul(o0, acc[NSUM - 1], Whole());
+                o0 = o1;
+                kt += KS;
+                if constexpr (PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // as after the prologue's
+            }
+        } else {
+            // the nk % 4 first tiles, to the sums after which the loop's passes start with acc[0]
+            auto single = [&](f32x16 (&sum)[NB][NBN]) {
+                load(kt + 1, o1, Free());
+                mul(o0, sum, Whole());
+                o0 = o1;
+                kt += 1;
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            };
+            if (rot == 1) single(acc[3]);
+            if (rot == 3) single(acc[1]);
+            if (rot >= 2) {
+                load(kt + 1, o1, Free());
+                mul(o0, acc[2], Whole());
+                load(kt + 2, o0, Free());
+                mul(o1, acc[3], Whole());
+                kt += 2;
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            }
         }
     }
-    for (; kt < nk; kt += 2 * KS) {
-        if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        __builtin_amdgcn_sched_barrier(0);
-        load(kt + KS, o1, Free());
-        mul(o0, acc[0], Whole());
-        interleave();
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        __builtin_amdgcn_sched_barrier(0);
-        load(kt + 2 * KS, o0, Free());
-        mul(o1, acc[NSUM - 1], Whole());
-        interleave();
-        __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NSUM < 4) {
+        for (; kt < nk; kt += 2 * KS) {
+            if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            __builtin_amdgcn_sched_barrier(0);
+            load(kt + KS, o1, Free());
+            mul(o0, acc[0], Whole());
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!PRECISE) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+            __builtin_amdgcn_sched_barrier(0);
+            load(kt + 2 * KS, o0, Free());
+            mul(o1, acc[NSUM - 1], Whole());
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+        auto step = [&](int next, Ops &into, const Ops &from, f32x16 (&sum)[NB][NBN]) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(next, into, Free());
+            mul(from, sum, Whole());
+            interleave();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (; kt < nk; kt += 4) {
+            step(kt + 1, o1, o0, acc[0]);
+            step(kt + 2, o0, o1, acc[1]);
+            step(kt + 3, o1, o0, acc[2]);
+            step(kt + 4, o0, o1, acc[3]);
+        }
     }
 
     PITON_PHASE(2);
@@ -910,10 +953,17 @@ void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
                     for (int r = 0; r < 16; r++) res[r] = res_of(i, j, r);
                 landed(res);
+                if constexpr (NSUM == 4) {  // acc[0] becomes the sum, in the order of the tiles' indexes
+                    const f32x16 s0 = acc[0][i][j], s1 = acc[1][i][j], s2 = acc[2][i][j], s3 = acc[3][i][j];
+                    acc[0][i][j] = rot == 0   ? ((s0 + s1) + s2) + s3
+                                   : rot == 1 ? ((s3 + s0) + s1) + s2
+                                   : rot == 2 ? ((s2 + s3) + s0) + s1
+                                              : ((s1 + s2) + s3) + s0;
+                }
                 auto put = [&](auto whole) {
 #pragma unroll
                     for (int r = 0; r < 16; r++)
-                        store(i, j, r, NSUM == 1 ? acc[0][i][j][r] : acc[0][i][j][r] + acc[NSUM - 1][i][j][r], bias[j],
+                        store(i, j, r, NSUM == 2 ? acc[0][i][j][r] + acc[NSUM - 1][i][j][r] : acc[0][i][j][r], bias[j],
                               res[r], whole);
                 };
                 if (whole_tile) put(std::true_type());
@@ -1243,12 +1293,14 @@ constexpr SplitForm kSplitForms[] = {
     {2, 4, 1, 2, 5.2f, {1.02f, 1.09f, 1.02f}, 8.0f, {12.f, 12.f, 12.f}},
     {2, 2, 1, 1, 3.4f, {1.02f, 1.14f, 1.02f}, 5.8f, {12.f, 12.f, 12.f}},
     {1, 1, 1, 2, 5.2f, {1.06f, 1.51f, 1.01f}, 0.0f, {12.5f, 10.5f, 10.8f}},
+    {1, 1, 1, 4, 5.2f, {1.06f, 1.51f, 1.01f}, 0.0f, {12.5f, 10.5f, 10.8f}},
     {2, 4, 4, 4, 1.2f, {1.04f, 1.12f, 1.07f}, 7.7f, {12.f, 12.f, 12.f}},
     {2, 2, 4, 4, 4.0f, {1.11f, 1.22f, 1.14f}, 2.4f, {12.f, 12.f, 12.f}},
     {1, 1, 4, 4, 4.2f, {1.39f, 1.59f, 1.56f}, 0.3f, {19.5f, 10.5f, 10.7f}},
 };
 constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
-constexpr int kSplitWide = 3;  // the index of <2, 4, 4>
+constexpr int kMaxSums = 4;
+constexpr int kSplitWide = 4;  // the index of <2, 4, 4>
 // tile rows per group of the entries that have no GROUP_SIZE_M: an XCD's tiles share B's columns
 // and A's rows in its L2 (2000 x 1000 x 784 36.5 us with groups of one row, 34.1 with 4 to 16)
 constexpr int kGroupRows = 8;
@@ -1269,14 +1321,30 @@ static float split_us(const SplitForm &f, int64_t M, int64_t N, int64_t K, int l
     if (f.ks == 1 && f.nbn < 4 && tiles > 2 * (int64_t)cus && rounds < 2) rounds = 2;
     const float wave = 0.432f * f.nb * f.nbn * (float)((nk + f.ks - 1) / f.ks);
     const float mb = (float)tiles * (float)nk * (f.nb + f.nbn) * 4096e-6f;
-    auto us = [&](int l) { return f.t0 + std::max((float)rounds * (wave * f.stretch[l] + f.round), mb / f.mbus[l]); };
+    // 32 x 32 tiles with four sums: three of the waves fit a SIMD (two sums: four), and the tiles past
+    // those run beside fewer (4000 x 950 x 260 26.8 us, 22.7 with two sums; 2000 x 1900 x 900 71.6, 64 x
+    // 64 tiles with four waves 62.6)
+    const float last = f.nb == 1 && f.ks == 1 && f.sums == 4 && tiles > 12 * (int64_t)cus ? 1.1f : 1.f;
+    auto us = [&](int l) {
+        return f.t0 + last * std::max((float)rounds * (wave * f.stretch[l] + f.round), mb / f.mbus[l]);
+    };
     return layout == kAnyLayout ? 0.5f * (us(0) + us(2)) : us(layout);
 }
-// the fastest form by the model, of those with `sums` partial sums (0: of all)
-static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int sums, float &us) {
+// The partial sums an element of a product keeps at least, as the waves that split K gave it when
+// they alone filled the chip: four below four 64 x 64 tiles per CU, two below eight, as long as
+// each has two K tiles. With half as many the error against float64 grows (inputs U[-1, 1], relative
+// 2-norm: 1971 x 654 x 1280 3.2e-7 with four and 4.5e-7 with two, 3897 x 2060 x 594 3.1e-7 with two
+// and 4.4e-7 with one).
+static int least_sums(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t tiles = split_tiles(SplitForm{2, 2}, M, N), nk = (K + 31) / 32;
+    const int by_tiles = tiles < 4 * (int64_t)cus ? 4 : tiles < 8 * (int64_t)cus ? 2 : 1;
+    return std::min(by_tiles, nk >= 8 ? 4 : nk >= 4 ? 2 : 1);
+}
+// the fastest form by the model, of those with `least` to `most` partial sums
+static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int least, int most, float &us) {
     int best = -1;
     for (int i = 0; i < kNumSplitForms; i++) {
-        if (sums && kSplitForms[i].sums != sums) continue;
+        if (kSplitForms[i].sums < least || kSplitForms[i].sums > most) continue;
         const float t = split_us(kSplitForms[i], M, N, K, layout, cus);
         if (best < 0 || t < us) best = i, us = t;
     }
@@ -1334,19 +1402,21 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule
     float us;
     if (nt > cus && ntw <= cus && nk >= 8 && nk <= 22) {
         // (column-major operands measured slower on it: the best of the others with four waves over K)
-        const int wide = wide_rule && p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, us);
+        const int wide = wide_rule && p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, 4, us);
         p.parts = 1;
         p.part[0] = SplitPart{wide, 0, 0, g.M, g.N};
         p.us = split_us(kSplitForms[wide], g.M, g.N, g.K, layout, cus);
         return p;
     }
     // the cut and the partial sums, by the model for no layout in particular
-    const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, sums, us);
+    const int least = sums ? sums : least_sums(g.M, g.N, g.K, cus), most = sums ? sums : kMaxSums;
+    const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, least, most, us);
     p.parts = 1;
     p.part[0] = SplitPart{form, 0, 0, g.M, g.N};
     float best = 0.97f * us;  // a second launch has to pay
     for (int i = 0; i < kNumSplitForms && !sums; i++) {
         const SplitForm &f = kSplitForms[i];
+        if (f.sums < least) continue;
         const int64_t tm = (g.M + 32 * f.nb - 1) / (32 * f.nb), tn = (g.N + 32 * f.nbn - 1) / (32 * f.nbn);
         const int64_t slots = 4 * (int64_t)cus / f.ks, full = tm * tn / slots * slots;
         const int64_t rows = full / tn, cols = full / tm;  // whole rows / columns of tiles in the full rounds
@@ -1355,7 +1425,7 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule
             if (dir ? cols <= 0 || N1 >= g.N : rows <= 0 || M1 >= g.M) continue;
             const int64_t M2 = dir ? g.M : g.M - M1, N2 = dir ? g.N - N1 : g.N;
             float rest;
-            const int form2 = best_form(M2, N2, g.K, kAnyLayout, cus, 0, rest);
+            const int form2 = best_form(M2, N2, g.K, kAnyLayout, cus, least, most, rest);
             const float t = split_us(f, M1, N1, g.K, kAnyLayout, cus) + rest;
             if (t < best) {
                 best = t;
@@ -1369,40 +1439,42 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule
     p.us = 0.f;
     for (int i = 0; i < p.parts; i++) {
         SplitPart &q = p.part[i];
-        q.form = best_form(q.M, q.N, g.K, layout, cus, kSplitForms[q.form].sums, us);
+        const int part_sums = kSplitForms[q.form].sums;
+        q.form = best_form(q.M, q.N, g.K, layout, cus, part_sums, part_sums, us);
         p.us += us;
     }
     return p;
 }
 
-// the recorded name of gemm_split_kernel<NB, NBN, KS, AM, BKC, TAIL>, with its parameters' values
-template <int NB, int NBN, int KS, int AM, bool BKC, bool TAIL>
+// the recorded name of gemm_split_kernel<NB, NBN, KS, AM, BKC, TAIL, NSUM>, with its parameters' values
+template <int NB, int NBN, int KS, int AM, bool BKC, bool TAIL, int NSUM>
 static const char *split_name() {
     static const std::string name = "gemm_split_kernel<" + std::to_string(NB) + ", " + std::to_string(NBN) + ", " +
                                     std::to_string(KS) + ", " +
                                     (AM == A_ROW16 ? "A_ROW16" : AM == A_ROW ? "A_ROW" : "A_COL") + ", " +
-                                    (BKC ? "true" : "false") + ", " + (TAIL ? "true" : "false") + ">";
+                                    (BKC ? "true" : "false") + ", " + (TAIL ? "true" : "false") + ", " +
+                                    std::to_string(NSUM) + ">";
     return name.c_str();
 }
 
-template <int NB, int NBN, int KS, int AM, bool BKC>
+template <int NB, int NBN, int KS, int NSUM, int AM, bool BKC>
 static void launch_split_one(const GemmArgs &g, unsigned tiles, hipStream_t st) {
-    if (g.K % (64 * KS) == 0)
-        PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, false>), (split_name<NB, NBN, KS, AM, BKC, false>()),
+    if (g.K % loop_k(KS, NSUM) == 0)
+        PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, false, NSUM>), (split_name<NB, NBN, KS, AM, BKC, false, NSUM>()),
                            dim3(tiles), dim3(64 * KS), 0, st, g);
     else
-        PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, true>), (split_name<NB, NBN, KS, AM, BKC, true>()),
+        PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, true, NSUM>), (split_name<NB, NBN, KS, AM, BKC, true, NSUM>()),
                            dim3(tiles), dim3(64 * KS), 0, st, g);
 }
 
-template <int NB, int NBN, int KS>
+template <int NB, int NBN, int KS, int NSUM>
 static void launch_split_ks(const GemmArgs &g, int am, bool bkc, unsigned tiles, hipStream_t st) {
-    if (am == A_ROW16 && !bkc) launch_split_one<NB, NBN, KS, A_ROW16, false>(g, tiles, st);
-    else if (am == A_ROW16) launch_split_one<NB, NBN, KS, A_ROW16, true>(g, tiles, st);
-    else if (am == A_ROW && !bkc) launch_split_one<NB, NBN, KS, A_ROW, false>(g, tiles, st);
-    else if (am == A_ROW) launch_split_one<NB, NBN, KS, A_ROW, true>(g, tiles, st);
-    else if (!bkc) launch_split_one<NB, NBN, KS, A_COL, false>(g, tiles, st);
-    else launch_split_one<NB, NBN, KS, A_COL, true>(g, tiles, st);
+    if (am == A_ROW16 && !bkc) launch_split_one<NB, NBN, KS, NSUM, A_ROW16, false>(g, tiles, st);
+    else if (am == A_ROW16) launch_split_one<NB, NBN, KS, NSUM, A_ROW16, true>(g, tiles, st);
+    else if (am == A_ROW && !bkc) launch_split_one<NB, NBN, KS, NSUM, A_ROW, false>(g, tiles, st);
+    else if (am == A_ROW) launch_split_one<NB, NBN, KS, NSUM, A_ROW, true>(g, tiles, st);
+    else if (!bkc) launch_split_one<NB, NBN, KS, NSUM, A_COL, false>(g, tiles, st);
+    else launch_split_one<NB, NBN, KS, NSUM, A_COL, true>(g, tiles, st);
 }
 
 static void launch_split(const GemmArgs &g, const SplitPlan &sp, int group_m, hipStream_t st) {
@@ -1421,12 +1493,13 @@ static void launch_split(const GemmArgs &g, const SplitPlan &sp, int group_m, hi
         gs.group_m = (int)(group_m > rows ? rows : group_m);
         gs.phase = phase_slot();
         const unsigned tiles = (unsigned)split_tiles(f, q.M, q.N);
-        if (f.nbn == 4 && f.ks == 4) launch_split_ks<2, 4, 4>(gs, sp.am, sp.bkc, tiles, st);
-        else if (f.nbn == 4) launch_split_ks<2, 4, 1>(gs, sp.am, sp.bkc, tiles, st);
-        else if (f.nb == 2 && f.ks == 4) launch_split_ks<2, 2, 4>(gs, sp.am, sp.bkc, tiles, st);
-        else if (f.nb == 2) launch_split_ks<2, 2, 1>(gs, sp.am, sp.bkc, tiles, st);
-        else if (f.ks == 4) launch_split_ks<1, 1, 4>(gs, sp.am, sp.bkc, tiles, st);
-        else launch_split_ks<1, 1, 1>(gs, sp.am, sp.bkc, tiles, st);
+        if (f.nbn == 4 && f.ks == 4) launch_split_ks<2, 4, 4, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nbn == 4) launch_split_ks<2, 4, 1, 2>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nb == 2 && f.ks == 4) launch_split_ks<2, 2, 4, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.nb == 2) launch_split_ks<2, 2, 1, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.ks == 4) launch_split_ks<1, 1, 4, 1>(gs, sp.am, sp.bkc, tiles, st);
+        else if (f.sums == 4) launch_split_ks<1, 1, 1, 4>(gs, sp.am, sp.bkc, tiles, st);
+        else launch_split_ks<1, 1, 1, 2>(gs, sp.am, sp.bkc, tiles, st);
     }
 }
 

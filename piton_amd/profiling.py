@@ -58,10 +58,10 @@ WORKLOADS = {
 # shape runs 240 wide tiles of 64 x 128)
 LAUNCHES = {
     ("gemm_direct_kernel<true, true, false, 4>", 65536): ("matmul 4096^3", 2),
-    ("gemm_split_kernel<1, 1, 4, 0, false, false>", 65536): ("matmul 512^3", 1),
-    ("gemm_split_kernel<2, 2, 4, 0, false, false>", 65536): ("matmul 1024^3", 1),
-    ("gemm_split_kernel<2, 4, 4, 1, false, true>", 61440): ("matmul 1000 x 1800 x 700 (row strides 703 / 1805 / 1807)", 1),
-    ("gemm_split_kernel<2, 2, 4, 0, true, false>", 65536): ("matmul 1024^3, B column-major", 1),
+    ("gemm_split_kernel<1, 1, 4, 0, false, false, 1>", 65536): ("matmul 512^3", 1),
+    ("gemm_split_kernel<2, 2, 4, 0, false, false, 1>", 65536): ("matmul 1024^3", 1),
+    ("gemm_split_kernel<2, 4, 4, 1, false, true, 1>", 61440): ("matmul 1000 x 1800 x 700 (row strides 703 / 1805 / 1807)", 1),
+    ("gemm_split_kernel<2, 2, 4, 0, true, false, 1>", 65536): ("matmul 1024^3, B column-major", 1),
     ("softmax_rows_kernel<4, true>", 262144): ("softmax 4096 x 1024", 1),
     ("softmax_wg_kernel<2, 512, true>", 2097152): ("softmax 4096 x 4096", 1),
     ("softmax_rows_kernel<8, false>", 196608): ("softmax 4096 x 1823", 1),

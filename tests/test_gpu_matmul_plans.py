@@ -72,3 +72,38 @@ def test_every_k_tail(M, N, tiles):
         for a_t, b_t, pad in ((False, False, 4), (False, False, 3), (True, False, 4), (False, True, 4 - K % 4)):
             got, names = _run(a, b, a_t, b_t, pad)
             assert torch.equal(got, want), (K, a_t, b_t, names)
+
+
+# the partial sums per element that the waves over K kept for these sizes: fewer than 1024 tiles of
+# 64 x 64 have four, fewer than 2048 two
+SUMS = [(1971, 654, 1280, 4), (1115, 2752, 354, 4), (2945, 960, 231, 4), (2112, 1664, 704, 4), (1024, 3353, 712, 4),
+        (3897, 2060, 594, 2), (2873, 2880, 620, 2), (3689, 2240, 2410, 2), (2578, 3130, 129, 2)]
+
+
+@pytest.mark.parametrize("M,N,K,sums", SUMS)
+def test_partial_sums_per_element(M, N, K, sums):
+    """Every form keeps at least `sums` interleaved partial sums, so the error against float64 is
+    that of sums so long: no larger than 1.1 times (the rounding errors are random: the relative
+    2-norm over 64 x N elements varies by 2 %) the error of the same sums formed one product after
+    another in float32; and four sums are the bits of four waves over K, which a product of 64 rows
+    has."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.rand(s, device="cuda", generator=g) * 2 - 1 for s in ((M, K), (K, N)))
+    got, names = _run(a, b, False, False, 4)
+    for name in names:  # gemm_split_kernel<.., .., waves over K, .., .., .., sums per wave>
+        values = name.rstrip(">").split(", ")
+        assert int(values[2]) * int(values[-1]) >= sums, names
+    rows = a[:64]
+    if sums == 4:
+        few, few_names = _run(rows, b, False, False, 4)
+        assert all(", 4, A_" in n for n in few_names), few_names
+        assert torch.equal(got[:64], few), (names, few_names)
+    part = torch.zeros((sums, 64, N), device="cuda")
+    for k in range(K):  # product by product, K tiles of 32 dealt to the sums
+        part[k // 32 % sums] += rows[:, k, None] * b[k]
+    chain = part[0]
+    for p in part[1:]:
+        chain = chain + p
+    want = rows.double() @ b.double()
+    err, ref = ((x.double() - want).norm().item() for x in (got[:64], chain))
+    assert err <= 1.1 * ref, (err, ref, names)
