@@ -1459,7 +1459,16 @@ static const char *split_name() {
 
 template <int NB, int NBN, int KS, int NSUM, int AM, bool BKC>
 static void launch_split_one(const GemmArgs &g, unsigned tiles, hipStream_t st) {
-    if (g.K % loop_k(KS, NSUM) == 0)
+    bool whole_passes = g.K % loop_k(KS, NSUM) == 0;
+    // 64 x 64 tiles of four waves, more than two to a CU: without a K tail the loop alone, which pads a
+    // wave's odd count of K tiles with a zero tile, since the workgroups of a CU then end one after
+    // the other and the third ones spread evenly; behind the tiles ahead of the loop they end together
+    // (829 x 3476 x 3264 190 -> 162 us, 1368 x 1920 x 3392 191 -> 164, 1344 x 1976 x 1600 99.5 -> 83.8;
+    // the other way about on unaligned rows, 1368 x 1920 x 1056 59.1 against 61.5, and on B
+    // column-major, 1344 x 1976 x 1600 101 against 112)
+    if constexpr (NB == 2 && NBN == 2 && KS == 4 && AM == A_ROW16 && !BKC)
+        whole_passes |= g.K % 32 == 0 && (int64_t)tiles > 2 * (int64_t)device_cu_count();
+    if (whole_passes)
         PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, false, NSUM>), (split_name<NB, NBN, KS, AM, BKC, false, NSUM>()),
                            dim3(tiles), dim3(64 * KS), 0, st, g);
     else

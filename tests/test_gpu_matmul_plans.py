@@ -34,7 +34,7 @@ def _run(a, b, a_t, b_t, pad, group=8):
 @pytest.mark.parametrize("M,N,K,launches", [(2500, 3000, 68, 1), (3000, 3200, 132, 1), (1100, 1800, 1000, 1),
                                             (700, 300, 44, 1), (33, 65, 4, 1), (2560, 2560, 2560, 2),
                                             (300, 4000, 3000, 2), (4000, 300, 3000, 2), (1, 1, 100, 1),
-                                            (2049, 2177, 96, 1)])
+                                            (2049, 2177, 96, 1), (1344, 1976, 1600, 1)])
 def test_forms_and_cuts(M, N, K, launches):
     """Every element within the float32 bound (K + 2) 2^-24 sum |a| |b| of float64; rows, columns
     and the padding (NaN) around them never reach C; all layouts and group orders agree bit for
@@ -107,3 +107,17 @@ def test_partial_sums_per_element(M, N, K, sums):
     want = rows.double() @ b.double()
     err, ref = ((x.double() - want).norm().item() for x in (got[:64], chain))
     assert err <= 1.1 * ref, (err, ref, names)
+
+
+@pytest.mark.parametrize("M,N,K,tail", [(1344, 1976, 1600, False), (829, 3476, 1632, False), (1000, 1000, 1632, True),
+                                        (1344, 1976, 1604, True)])
+def test_zero_tiles_pad_odd_counts(M, N, K, tail):
+    """64 x 64 tiles, more than two to a CU, and no K tail: every wave takes its K tiles in pairs,
+    the last one of an odd count beside a tile of zeros; others take it ahead of the loop. Dyadic
+    inputs with NaN around them: float64's bits."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randint(-4, 5, s, device="cuda", generator=g).float() / 4 for s in ((M, K), (K, N)))
+    got, (name, *_) = _run(a, b, False, False, 4)
+    assert torch.equal(got, (a.double() @ b.double()).float())
+    if rt.device_info()["cu_count"] == 256:
+        assert name == f"gemm_split_kernel<2, 2, 4, A_ROW16, false, {str(tail).lower()}, 1>"
