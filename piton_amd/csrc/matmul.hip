@@ -1300,7 +1300,6 @@ constexpr SplitForm kSplitForms[] = {
 };
 constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
 constexpr int kMaxSums = 4;
-constexpr int kSplitWide = 4;  // the index of <2, 4, 4>
 // tile rows per group of the entries that have no GROUP_SIZE_M: an XCD's tiles share B's columns
 // and A's rows in its L2 (2000 x 1000 x 784 36.5 us with groups of one row, 34.1 with 4 to 16)
 constexpr int kGroupRows = 8;
@@ -1369,7 +1368,7 @@ struct SplitPlan {
     float us;
 };
 // sums: 0, or the partial sums every element must have (one launch then, without a cut).
-static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule) {
+static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
     SplitPlan p{0, {}, 0, false, 0.f};
     if (g.K <= 0 || g.M <= 0 || g.N <= 0) return p;
     // A with stride 1 along K (16-byte loads where its rows are 16-byte aligned and K % 4 == 0) or
@@ -1390,24 +1389,7 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums, bool wide_rule
         split_tiles(SplitForm{1, 1}, g.M, g.N) > 0x7FFFFFFF)
         return p;
     const int layout = p.bkc ? 2 : p.am == A_ROW ? 1 : 0;
-    // the wide tile with four waves over K: where 64 x 64 tiles would put two workgroups on some CUs
-    // and 64 x 128 ones fit one per CU, up to 22 K tiles. It was the best form there when its
-    // square tiles held an address per k and ran one wave per SIMD; now 32 x 32 tiles measure
-    // faster on aligned rows (2048 x 768 x 256 13.1 against 16.4 us) and the same on unaligned ones
-    // (1000 x 1800 x 700, 33.5 against 33.1), and past 22 tiles the model chooses (2000 x 1000 x 784
-    // 35.4 -> 31.9). The rule stays for the matmul entry (wide_rule), whose tests hold these shapes
-    // to it.
-    const int64_t nt = split_tiles(SplitForm{2, 2}, g.M, g.N), ntw = split_tiles(SplitForm{2, 4}, g.M, g.N);
-    const int64_t nk = (g.K + 31) / 32;
     float us;
-    if (nt > cus && ntw <= cus && nk >= 8 && nk <= 22) {
-        // (column-major operands measured slower on it: the best of the others with four waves over K)
-        const int wide = wide_rule && p.am != A_COL && !p.bkc ? kSplitWide : best_form(g.M, g.N, g.K, layout, cus, 4, 4, us);
-        p.parts = 1;
-        p.part[0] = SplitPart{wide, 0, 0, g.M, g.N};
-        p.us = split_us(kSplitForms[wide], g.M, g.N, g.K, layout, cus);
-        return p;
-    }
     // the cut and the partial sums, by the model for no layout in particular
     const int least = sums ? sums : least_sums(g.M, g.N, g.K, cus), most = sums ? sums : kMaxSums;
     const int form = best_form(g.M, g.N, g.K, kAnyLayout, cus, least, most, us);
@@ -1545,7 +1527,7 @@ static void launch_direct(bool one_gen, bool wide, bool akc, bool bkc, const Gem
 // Whole tiles that fill whole generations take the direct kernel, other shapes the split kernel when
 // each operand has stride 1 along one axis, the rest the LDS kernel. sums: 0, or the partial sums
 // an element must have (plan_split): then the split kernel alone, wherever it applies.
-static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums, bool wide_rule) {
+static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
     if (g.M == 0 || g.N == 0) return PITON_OK;
     const int64_t tiles = sat_mul((g.M + GBM - 1) / GBM, (g.N + GBN - 1) / GBN);
     PITON_REQUIRE(tiles <= 0x7FFFFFFF, PITON_EUNSUPPORTED, "%s: %lld tiles exceed one grid", what, (long long)tiles);
@@ -1584,7 +1566,7 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums, b
     // (3072^3, 2.25 generations: 540 -> 433 us)
     const int64_t dgens = gens(dtiles);
     const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
-    const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums, wide_rule) : SplitPlan{};
+    const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums) : SplitPlan{};
     const float direct_us = 4.f + dgens * (0.432f * (g.K / 32) * (wide ? 8 : 4) * 1.02f + (wide ? 8.f : 6.f));
     if (sp.parts > 0 && (sums || !(direct && ntiles >= cus && direct_us <= sp.us))) {
         launch_split(g, sp, group_user, st);
@@ -1630,7 +1612,7 @@ int32_t piton_mi355x_matmul(const float *a, const float *b, float *c, int64_t M,
     if (rc) return rc;
     GemmArgs g{a, b, c, M, N, K, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
                group_size_m, nullptr, 0, nullptr, 0, 0, 0};
-    rc = launch_gemm(g, (hipStream_t)stream, "matmul", 0, true);
+    rc = launch_gemm(g, (hipStream_t)stream, "matmul", 0);
     if (rc == PITON_OK) clear_error();
     return rc;
 }
@@ -1662,13 +1644,13 @@ int32_t piton_mi355x_dense(const float *x, const float *w, const float *bias, fl
             g.M = std::min(M - m, kDenseChainRows);
             g.a = x + m * K;
             g.c = y + m * N;
-            rc = launch_gemm(g, st, "dense", kDenseChainSums, false);
+            rc = launch_gemm(g, st, "dense", kDenseChainSums);
         }
     } else if (M > 0 && M <= 64 && small_m_fast(g) && (N + SMN - 1) / SMN <= 0x7FFFFFFF) {
         launch_small_m<false>(g, small_m_grid(g), dim3(64 * SMWAVES), st);
         rc = check_launch("dense");
     } else {
-        rc = launch_gemm(g, st, "dense", 0, false);
+        rc = launch_gemm(g, st, "dense", 0);
     }
     if (rc) return rc;
     if (argmax_out && M > 0) {
@@ -1706,7 +1688,7 @@ int32_t piton_mi355x_linear(const float *x, int64_t ldx, const float *w, const f
             PITON_LAUNCH((gemm_small_m_kernel<false, false>), grid, block, 0, (hipStream_t)stream, g);
         rc = check_launch("linear");
     } else {
-        rc = launch_gemm(g, (hipStream_t)stream, "linear", 0, false);
+        rc = launch_gemm(g, (hipStream_t)stream, "linear", 0);
     }
     if (rc == PITON_OK) clear_error();
     return rc;

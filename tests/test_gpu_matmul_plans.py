@@ -121,3 +121,19 @@ def test_zero_tiles_pad_odd_counts(M, N, K, tail):
     assert torch.equal(got, (a.double() @ b.double()).float())
     if rt.device_info()["cu_count"] == 256:
         assert name == f"gemm_split_kernel<2, 2, 4, A_ROW16, false, {str(tail).lower()}, 1>"
+
+
+@pytest.mark.parametrize("M,N,K", [(900, 1500, 260), (1767, 896, 256), (2176, 512, 308), (1000, 1800, 700)])
+def test_matmul_linear_and_dense_take_the_same_form(M, N, K):
+    """One planner for the three entries: the same product gets the same launches and bits from each."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = (torch.rand(s, device="cuda", generator=g) * 2 - 1 for s in ((M, K), (K, N)))
+    c, y, z = (torch.full((M, N), -7.0, device="cuda") for _ in range(3))
+    names = []
+    for call in (lambda: rt.matmul(a, b, c, M, N, K, K, 1, N, 1, N, 1, 8),
+                 lambda: rt.linear(a, K, b, None, None, 0, y, N, M, N, K),
+                 lambda: rt.dense(a, b, None, z, M, N, K, add_bias=False)):
+        call()
+        names.append([x["kernel"] for x in rt.last_launches()])
+    assert names[0] == names[1] == names[2], names
+    assert torch.equal(c, y) and torch.equal(c, z)
