@@ -1278,25 +1278,27 @@ static int layout_b(const GemmArgs &g) {
 //     of 32 x 32 x 32 takes 0.432 us (16 MFMAs of 64 clocks at 2.37 GHz);
 //   * the operand bytes the waves load over what the L2s deliver (`mbus`, MB per us), which bounds
 //     the 32 x 32 tiles (half the products per byte of the 64 x 64 ones);
-// each by layout: 16-byte rows, A's rows unaligned, B column-major. Fitted to 78 shapes from 80 x 64
-// x 120 to 2560^3 in every form, three operand sets in turn (4-7 % rms); taking the form it names
-// costs 1.4 % on average against the best one measured. The rule before (tiles of 64 from as many of
+// each by layout: 16-byte rows, A's rows unaligned, B column-major, and between the first and the third
+// for what is to depend on the sizes alone. Fitted to 78 shapes from 80 x 64
+// x 120 to 2560^3 in every form, three operand sets in turn (4-7 % rms), the rates of 32 x 32 tiles with
+// B column-major to 30 more (10.8 and 10.7 MB per us at first: 3324 x 1664 x 384 took 67.6 us against
+// 59); taking the form it names costs 2 % on average against the best one measured. The rule before (tiles of 64 from as many of
 // them as CUs, waves doubled up to eight per CU) cost 6.5 %: 1536^3 82.6 -> 71.1 us, 2697 x 1640 x
 // 2428 233 -> 203, 128 x 340 x 200 6.5 -> 5.5. Two waves over K are left out: the two such
 // workgroups of a CU ran one after the other (1330 x 212 x 3772 57 us against 52 with four).
 // `sums`: the interleaved partial sums of an element's K tiles; forms with as many add alike.
 struct SplitForm {
     int nb, nbn, ks, sums;
-    float t0, stretch[3], round, mbus[3];
+    float t0, stretch[4], round, mbus[4];
 };
 constexpr SplitForm kSplitForms[] = {
-    {2, 4, 1, 2, 5.2f, {1.02f, 1.09f, 1.02f}, 8.0f, {12.f, 12.f, 12.f}},
-    {2, 2, 1, 1, 3.4f, {1.02f, 1.14f, 1.02f}, 5.8f, {12.f, 12.f, 12.f}},
-    {1, 1, 1, 2, 5.2f, {1.06f, 1.51f, 1.01f}, 0.0f, {12.5f, 10.5f, 10.8f}},
-    {1, 1, 1, 4, 5.2f, {1.06f, 1.51f, 1.01f}, 0.0f, {12.5f, 10.5f, 10.8f}},
-    {2, 4, 4, 4, 1.2f, {1.04f, 1.12f, 1.07f}, 7.7f, {12.f, 12.f, 12.f}},
-    {2, 2, 4, 4, 4.0f, {1.11f, 1.22f, 1.14f}, 2.4f, {12.f, 12.f, 12.f}},
-    {1, 1, 4, 4, 4.2f, {1.39f, 1.59f, 1.56f}, 0.3f, {19.5f, 10.5f, 10.7f}},
+    {2, 4, 1, 2, 5.2f, {1.02f, 1.09f, 1.02f, 1.02f}, 8.0f, {12.f, 12.f, 12.f, 12.f}},
+    {2, 2, 1, 1, 3.4f, {1.02f, 1.14f, 1.02f, 1.02f}, 5.8f, {12.f, 12.f, 12.f, 12.f}},
+    {1, 1, 1, 2, 5.2f, {1.06f, 1.51f, 1.01f, 1.035f}, 0.0f, {12.5f, 10.5f, 9.5f, 11.59f}},
+    {1, 1, 1, 4, 5.2f, {1.06f, 1.51f, 1.01f, 1.035f}, 0.0f, {12.5f, 10.5f, 9.5f, 11.59f}},
+    {2, 4, 4, 4, 1.2f, {1.04f, 1.12f, 1.07f, 1.055f}, 7.7f, {12.f, 12.f, 12.f, 12.f}},
+    {2, 2, 4, 4, 4.0f, {1.11f, 1.22f, 1.14f, 1.125f}, 2.4f, {12.f, 12.f, 12.f, 12.f}},
+    {1, 1, 4, 4, 4.2f, {1.39f, 1.59f, 1.56f, 1.475f}, 0.3f, {19.5f, 10.5f, 8.7f, 13.82f}},
 };
 constexpr int kNumSplitForms = sizeof kSplitForms / sizeof kSplitForms[0];
 constexpr int kMaxSums = 4;
@@ -1309,25 +1311,26 @@ constexpr int64_t kDenseChainRows = 1 << 20;     // rows of up to 256 floats wit
 static int64_t split_tiles(const SplitForm &f, int64_t M, int64_t N) {
     return sat_mul((M + 32 * f.nb - 1) / (32 * f.nb), (N + 32 * f.nbn - 1) / (32 * f.nbn));
 }
-constexpr int kAnyLayout = -1;  // the mean of aligned rows and B column-major
+constexpr int kAnyLayout = 3;
 static float split_us(const SplitForm &f, int64_t M, int64_t N, int64_t K, int layout, int cus) {
     const int64_t slots = 4 * (int64_t)cus / f.ks, nk = (K + 31) / 32;
     const int64_t tiles = split_tiles(f, M, N);
-    int64_t rounds = (tiles + slots - 1) / slots;
     // workgroups of one wave where two fit a SIMD: the dispatcher does not spread one round of them
     // evenly (1023 tiles of 64 x 64 on 1024 SIMDs took 150 or 282 us, depending on what ran before;
-    // as workgroups of four waves with a tile each, full rounds of them took 10 % longer)
-    if (f.ks == 1 && f.nbn < 4 && tiles > 2 * (int64_t)cus && rounds < 2) rounds = 2;
+    // as workgroups of four waves with a tile each, full rounds of them took 10 % longer), nor a third
+    // or fourth one of 64 x 64 tiles (4032 x 3072 x 1000, 2.95 rounds, took 3.75 rounds' time, 16 such
+    // shapes 2.7 to 3.8; 3392 x 4992 x 1000, four, 4.8)
+    float rounds = (float)((tiles + slots - 1) / slots);
+    if (f.ks == 1 && f.nbn < 4 && tiles > 2 * (int64_t)cus && rounds < 2.f) rounds = 2.f;
+    if (f.ks == 1 && f.nbn == 2 && rounds > 2.f) rounds += 0.4f;
     const float wave = 0.432f * f.nb * f.nbn * (float)((nk + f.ks - 1) / f.ks);
     const float mb = (float)tiles * (float)nk * (f.nb + f.nbn) * 4096e-6f;
     // 32 x 32 tiles with four sums: three of the waves fit a SIMD (two sums: four), and the tiles past
     // those run beside fewer (4000 x 950 x 260 26.8 us, 22.7 with two sums; 2000 x 1900 x 900 71.6, 64 x
     // 64 tiles with four waves 62.6)
     const float last = f.nb == 1 && f.ks == 1 && f.sums == 4 && tiles > 12 * (int64_t)cus ? 1.1f : 1.f;
-    auto us = [&](int l) {
-        return f.t0 + last * std::max((float)rounds * (wave * f.stretch[l] + f.round), mb / f.mbus[l]);
-    };
-    return layout == kAnyLayout ? 0.5f * (us(0) + us(2)) : us(layout);
+    const float us = f.t0 + last * std::max(rounds * (wave * f.stretch[layout] + f.round), mb / f.mbus[layout]);
+    return f.sums == 1 ? 1.02f * us : us;  // of forms as fast, the one with more partial sums
 }
 // The partial sums an element of a product keeps at least, as the waves that split K gave it when
 // they alone filled the chip: four below four 64 x 64 tiles per CU, two below eight, as long as
@@ -1352,7 +1355,7 @@ static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int l
 
 // A product as one launch, or as two: whole rounds of one form over the first rows (columns) of C
 // and the rest in the form that suits it, where the model finds that faster than letting a last
-// round run part full (2560^3 296 -> 269 us, 300 x 4000 x 3000 94 -> 73). parts 0: the split
+// round run part full (2560^3 296 -> 269 us, 300 x 4000 x 3000 99.9 -> 68.4). parts 0: the split
 // kernel does not apply. The cut and the partial sums depend on the sizes alone, so every layout of
 // A and B (and every group order) adds each element's products in the same order and gives the
 // same bits.
@@ -1442,14 +1445,18 @@ static const char *split_name() {
 template <int NB, int NBN, int KS, int NSUM, int AM, bool BKC>
 static void launch_split_one(const GemmArgs &g, unsigned tiles, hipStream_t st) {
     bool whole_passes = g.K % loop_k(KS, NSUM) == 0;
-    // 64 x 64 tiles of four waves, more than two to a CU: without a K tail the loop alone, which pads a
-    // wave's odd count of K tiles with a zero tile, since the workgroups of a CU then end one after
-    // the other and the third ones spread evenly; behind the tiles ahead of the loop they end together
-    // (829 x 3476 x 3264 190 -> 162 us, 1368 x 1920 x 3392 191 -> 164, 1344 x 1976 x 1600 99.5 -> 83.8;
-    // the other way about on unaligned rows, 1368 x 1920 x 1056 59.1 against 61.5, and on B
-    // column-major, 1344 x 1976 x 1600 101 against 112)
-    if constexpr (NB == 2 && NBN == 2 && KS == 4 && AM == A_ROW16 && !BKC)
-        whole_passes |= g.K % 32 == 0 && (int64_t)tiles > 2 * (int64_t)device_cu_count();
+    // 64 x 64 tiles of four waves, two to three to a CU: without a K tail the loop alone, which pads a
+    // wave's odd count of K tiles (from 13 on: a zero tile costs its share) with a zero tile, since
+    // the workgroups of a CU then end one after the other and the third ones spread evenly; behind the
+    // tiles ahead of the loop they end together (829 x 3476 x 3264 190 -> 162 us, 1368 x 1920 x 3392
+    // 191 -> 164, 1344 x 1976 x 1600 99.5 -> 83.8; with more to a CU it is the other way about, 4461 x
+    // 1344 x 1984 184 -> 208, as on unaligned rows, 1368 x 1920 x 1056 59.1 -> 61.5, and on B
+    // column-major, 1344 x 1976 x 1600 101 -> 112)
+    if constexpr (NB == 2 && NBN == 2 && KS == 4 && AM == A_ROW16 && !BKC) {
+        const int64_t cus = device_cu_count();
+        whole_passes |= g.K % 32 == 0 && tiles > 2 * cus && tiles <= 3 * cus &&
+                        (g.K > 12 * 128 || (g.K + 127) / 128 % 2 == 0);
+    }
     if (whole_passes)
         PITON_LAUNCH_NAMED((gemm_split_kernel<NB, NBN, KS, AM, BKC, false, NSUM>), (split_name<NB, NBN, KS, AM, BKC, false, NSUM>()),
                            dim3(tiles), dim3(64 * KS), 0, st, g);

@@ -137,3 +137,16 @@ def test_matmul_linear_and_dense_take_the_same_form(M, N, K):
         names.append([x["kernel"] for x in rt.last_launches()])
     assert names[0] == names[1] == names[2], names
     assert torch.equal(c, y) and torch.equal(c, z)
+
+
+@pytest.mark.parametrize("M,N,K", [(3324, 1664, 384), (1971, 654, 1280), (4032, 3072, 1000)])
+def test_forms_of_slow_rounds_are_left(M, N, K):
+    """B column-major with many 32 x 32 tiles of one wave, and a third round of 64 x 64 tiles of one wave,
+    take longer than whole rounds of another form, which the planner takes instead."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.randint(-4, 5, s, device="cuda", generator=g).float() / 4 for s in ((M, K), (K, N)))
+    got, names = _run(a, b, False, True, 4)
+    assert torch.equal(got, (a.double() @ b.double()).float())
+    if rt.device_info()["cu_count"] == 256:
+        slow = "<2, 2, 1," if M == 4032 else "<1, 1, 1,"
+        assert all(slow not in n for n in names), names
