@@ -1356,9 +1356,11 @@ static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int l
 // A product as one launch, or as two: whole rounds of one form over the first rows (columns) of C
 // and the rest in the form that suits it, where the model finds that faster than letting a last
 // round run part full (2560^3 296 -> 269 us, 300 x 4000 x 3000 99.9 -> 68.4). parts 0: the split
-// kernel does not apply. The cut and the partial sums depend on the sizes alone, so every layout of
-// A and B (and every group order) adds each element's products in the same order and gives the
-// same bits.
+// kernel does not apply. The cut and the partial sums depend on the sizes alone, and so does `us`, the
+// time that launch_gemm holds against the direct kernel's: every layout of A and B (and every group
+// order) of one of the two kernels adds each element's products in the same order and gives the same
+// bits, and operands that both kernels take go to the same one (768 x 7936 x 256 with B column-major, the
+// split kernel's slower side, 42.2 us, the direct kernel 41.2).
 struct SplitPart {
     int form;
     int64_t m0, n0, M, N;
@@ -1368,7 +1370,7 @@ struct SplitPlan {
     SplitPart part[2];
     int am;    // SplitA: A's layout
     bool bkc;  // B column-major
-    float us;
+    float us;  // by the model, for aligned rows whatever the layout
 };
 // sums: 0, or the partial sums every element must have (one launch then, without a cut).
 static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
@@ -1425,8 +1427,9 @@ static SplitPlan plan_split(const GemmArgs &g, int cus, int sums) {
     for (int i = 0; i < p.parts; i++) {
         SplitPart &q = p.part[i];
         const int part_sums = kSplitForms[q.form].sums;
-        q.form = best_form(q.M, q.N, g.K, layout, cus, part_sums, part_sums, us);
+        best_form(q.M, q.N, g.K, 0, cus, part_sums, part_sums, us);
         p.us += us;
+        q.form = best_form(q.M, q.N, g.K, layout, cus, part_sums, part_sums, us);
     }
     return p;
 }

@@ -150,3 +150,20 @@ def test_forms_of_slow_rounds_are_left(M, N, K):
     if rt.device_info()["cu_count"] == 256:
         slow = "<2, 2, 1," if M == 4032 else "<1, 1, 1,"
         assert all(slow not in n for n in names), names
+
+
+# whole 128 x 128 tiles in generations that are part full: the split kernel's and the direct kernel's
+# times lie closest together here
+@pytest.mark.parametrize("M,N,K", [(768, 7936, 256), (1280, 5120, 256), (5888, 1024, 256), (5888, 2560, 128),
+                                   (1664, 3840, 256), (2688, 6144, 128)])
+def test_whole_tiles_take_one_kernel_in_every_layout(M, N, K):
+    """The choice between the split and the direct kernel depends on the sizes alone, so A and B stored
+    either way give the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, b = (torch.rand(s, device="cuda", generator=g) * 2 - 1 for s in ((M, K), (K, N)))
+    base, names = _run(a, b, False, False, 4)
+    family = {n.partition("<")[0] for n in names}
+    for a_t, b_t in ((True, False), (False, True), (True, True)):
+        got, names = _run(a, b, a_t, b_t, 4)
+        assert {n.partition("<")[0] for n in names} == family, (a_t, b_t, names)
+        assert torch.equal(got, base), (a_t, b_t, names)
