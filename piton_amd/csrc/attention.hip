@@ -918,12 +918,15 @@ template <int D>
 constexpr int kDecodeChunk = 16384 / D;
 
 template <int D, bool VEC>
-__global__ __launch_bounds__(256) void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC ? 4 : 1)))
+void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
     constexpr int DCH = kDecodeChunk<D>, LPR = D / 4, KG = 256 / LPR, NR = DCH / KG;
     static_assert(NR == 16, "16 float4 of K and of V per thread");
     __shared__ float red[8];
     __shared__ __attribute__((aligned(16))) float part[KG][D];
+    __shared__ int large;
     const int t = threadIdx.x;
+    if (t == 0) large = 0;
     const int nbh = gridDim.x / nsplit, bh = blockIdx.x % nbh, chunk = blockIdx.x / nbh;
     const int64_t b = bh / g.n_heads, h = bh % g.n_heads;
     const int key0 = chunk * DCH, n = min(DCH, g.n_keys - key0);
@@ -966,7 +969,7 @@ __global__ __launch_bounds__(256) void attn_decode_part(DecodeArgs g, float *ws,
         sc[i] = i * KG + kg < n ? s : -INFINITY;
         mloc = fmaxf(mloc, sc[i]);
     }
-    const float m = block_reduce4(mloc, MaxOp(), red);
+    float m = block_reduce4(mloc, MaxOp(), red);
     PITON_PHASE(2);
     const float mref = m == -INFINITY ? 0.f : m;  // a chunk of -inf scores alone: every weight 0
     float lsum = 0.f;
@@ -979,13 +982,26 @@ __global__ __launch_bounds__(256) void attn_decode_part(DecodeArgs g, float *ws,
 #pragma unroll
         for (int i = 0; i < NR; i++)
             if (i * KG + kg >= n) vv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // the lane group's part of P V, the weights times `scale`
+    auto add_up = [&](float scale) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < NR; i++)
+        for (int i = 0; i < NR; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[e] = fmaf(sc[i], vv[i][e], acc[e]);
-    *reinterpret_cast<f32x4 *>(&part[kg][4 * dq]) = acc;
-    const float l = block_reduce4(dq == 0 ? lsum : 0.f, SumOp(), red + 4);  // its barrier publishes the sums
+            for (int e = 0; e < 4; e++) acc[e] = fmaf(sc[i] * scale, vv[i][e], acc[e]);
+        *reinterpret_cast<f32x4 *>(&part[kg][4 * dq]) = acc;
+        return fmaxf(fmaxf(fabsf(acc.x), fabsf(acc.y)), fmaxf(fabsf(acc.z), fabsf(acc.w)));
+    };
+    if (add_up(1.f) >= 0x1p121f) large = 1;
+    float l = block_reduce4(dq == 0 ? lsum : 0.f, SumOp(), red + 4);  // its barrier publishes the sums
+    // values that take a chunk's sum near the largest float, which the whole softmax may give little
+    // weight or none: the chunk leaves its sums 2^-9 as large under a maximum 9 higher
+    if (nsplit > 1 && large) {
+        add_up(0x1p-9f);
+        __syncthreads();
+        m += 9.f;
+        l *= 0x1p-9f;
+    }
     float v = 0.f;
     if (t < D) {
         v = part[0][t];

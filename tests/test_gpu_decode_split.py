@@ -88,6 +88,25 @@ def test_masked_and_infinite_keys():
     assert np.isposinf(got[0, 2, 7]) and np.isfinite(np.delete(got[0, 2], 7)).all()
 
 
+@pytest.mark.parametrize("dh,n", [(64, 600), (128, 300), (32, 1100)])
+def test_large_values_of_keys_without_weight(dh, n):
+    """Finite values near the largest float whose keys have a weight of 0, or next to it, beside the
+    others: their chunk's own sum would overflow, the result is float64's within the float32 bound."""
+    q, k, v = _cache(1, 2, n, dh, 0, dh + n)
+    chunk = 16384 // dh
+    q[...], k[...] = 1, 0
+    k[:chunk, :, 0] = -dh * 0.5   # head 0: the first chunk's weights underflow
+    k[:chunk, :, 1] = -2.0        # head 1: they are 2^-(2 dh log2 e) and smaller, and count
+    v[:chunk] = np.float32(1e37) * np.sign(v[:chunk])
+    v[:chunk, :, 1] *= np.float32(1e-20)
+    got, parts, _ = _split(q, k, v, 1.0)
+    assert parts > 1
+    ref = _fp64(q, k, v, 1.0)
+    assert np.isfinite(got).all()
+    for h in range(2):
+        assert fp64.rel_fro(got[:, h], ref[:, h]) <= 1e-5, h
+
+
 def test_captured_calls_replay():
     """The workspace of a captured call belongs to the graph: replays with eager calls of other
     shapes between them give the eager bits."""
