@@ -899,9 +899,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs g) {
     }
 }
 
-// The cache in chunks of DCH keys, one workgroup per (batch, head) and chunk: workgroup (bh, c)
-// attends head bh's query to the keys of chunk c. A single chunk stores the output; several leave
-// (m, l, O) unnormalised in the caller's workspace and attn_decode_merge adds them. Bound by HBM:
+// The cache in chunks, one workgroup per (batch, head) and chunk: workgroup (bh, c) attends head
+// bh's query to the keys of chunk c. A single chunk stores the output; several leave (m, l, O)
+// unnormalised in the caller's workspace and attn_decode_merge adds them. Where the heads fill the
+// chip, one workgroup takes up to three chunks' keys itself, eight rows at a time. Bound by HBM:
 // attn_decode_kernel's one workgroup per head is a serial chain of key loads (64 heads x 4096
 // keys of 64: 64 of 256 CUs, 160 us, 0.84 TB/s); the chunks fill the chip and each workgroup
 // requests its 64 KB of K and V before it uses any of it (25 us, 5.4 TB/s with the merge; 6.3
@@ -912,27 +913,29 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs g) {
 //   * lane group kg scores the keys i * KG + kg it also adds to P V, so the weights never leave
 //     its registers; a key's dot product adds over the group by lane exchanges;
 //   * the chunk is sized so that a thread holds 16 float4 of K and 16 of V whatever D is; a cache of
-//     one chunk loads as many rows per thread as its keys need (NR, a power of two): 704 heads of 32
-//     with 12 keys took 6.8 us with 16 rows and 5.4 with one wave's;
+//     one chunk loads as many rows per thread as its keys need (NR, a power of two): 256 heads of 64
+//     with 8 keys 4.33 -> 2.83 us, with 100 keys 4.37 -> 3.32, of 128 with 8 keys 4.53 -> 2.79;
 //   * keys past n_keys load the last key's row (in bounds for any strides) and drop out by a score
 //     of -inf and a zeroed V, so an infinity in that row counts once.
 template <int D>
 constexpr int kDecodeChunk = 16384 / D;
 constexpr int kDecodeRows = 16;
 
-template <int D, bool VEC, int NR>
+// NCH: the chunks of NR rows that a workgroup takes; 0: one of a cache split over several workgroups
+template <int D, bool VEC, int NR, int NCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC ? 4 : 1)))
 void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
-    constexpr int LPR = D / 4, KG = 256 / LPR, DCH = NR * KG;
-    static_assert(NR < kDecodeRows || DCH == kDecodeChunk<D>, "a chunk fills kDecodeRows rows");
+    constexpr bool SPLIT = NCH == 0;
+    constexpr int LPR = D / 4, KG = 256 / LPR, DCH = NR * KG, CH = SPLIT ? 1 : NCH;
+    static_assert(NR < kDecodeRows ? !SPLIT : DCH == kDecodeChunk<D> && CH == 1, "a chunk fills kDecodeRows rows");
     __shared__ float red[8];
     __shared__ __attribute__((aligned(16))) float part[KG][D];
     __shared__ int large;
     const int t = threadIdx.x;
-    if (t == 0) large = 0;
-    const int nbh = gridDim.x / nsplit, bh = blockIdx.x % nbh, chunk = blockIdx.x / nbh;
+    if (SPLIT && t == 0) large = 0;
+    const int nbh = SPLIT ? gridDim.x / nsplit : gridDim.x, bh = blockIdx.x % nbh, chunk = blockIdx.x / nbh;
     const int64_t b = bh / g.n_heads, h = bh % g.n_heads;
-    const int key0 = chunk * DCH, n = min(DCH, g.n_keys - key0);
+    const int key0 = chunk * DCH, n = min(CH * DCH, g.n_keys - key0);
     const int dq = t % LPR, kg = t / LPR;
     const bool d_ok = 4 * dq < g.head_dim;  // head_dim is a multiple of 16
     const int d0 = d_ok ? 4 * dq : 0;
@@ -948,58 +951,78 @@ void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
         else return f32x4{r[0], r[1], r[2], r[3]};
     };
     f32x4 kv[NR], vv[NR];
+    auto load = [&](f32x4 (&x)[NR], const float *p, int64_t stride, int c) {
+#pragma unroll
+        for (int i = 0; i < NR; i++) x[i] = row4(p + (int64_t)(key0 + min(c * DCH + i * KG + kg, n - 1)) * stride);
+    };
     f32x4 q4 = f32x4{qp[0], qp[1], qp[2], qp[3]};
-#pragma unroll
-    for (int i = 0; i < NR; i++) kv[i] = row4(kp + (int64_t)(key0 + min(i * KG + kg, n - 1)) * g.s_kn);
-#pragma unroll
-    for (int i = 0; i < NR; i++) vv[i] = row4(vp + (int64_t)(key0 + min(i * KG + kg, n - 1)) * g.s_vn);
+    load(kv, kp, g.s_kn, 0);
+    if constexpr (CH == 1) load(vv, vp, g.s_vn, 0);
 #pragma unroll
     for (int e = 0; e < 4; e++) q4[e] = d_ok ? q4[e] * g.scale : 0.f;
 
     PITON_PHASE_WAIT_LOADS();
     PITON_PHASE(1);
-    float sc[NR], mloc = -INFINITY;
+    float sc[CH][NR], mloc = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < NR; i++) {
-        float s = 0.f;
+    for (int c = 0; c < CH; c++) {
+        if (c > 0 && c * DCH >= n) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) s = d_ok ? fmaf(q4[e], kv[i][e], s) : 0.f;
-        s += dpp_f<DPP_QUAD_XOR1>(s);
-        s += dpp_f<DPP_QUAD_XOR2>(s);
-        s += dpp_f<DPP_ROW_HALF_MIRROR>(s);
-        if constexpr (LPR >= 16) s += dpp_f<DPP_ROW_MIRROR>(s);
-        if constexpr (LPR >= 32) s += __shfl_xor(s, 16);
-        sc[i] = i * KG + kg < n ? s : -INFINITY;
-        mloc = fmaxf(mloc, sc[i]);
+            for (int i = 0; i < NR; i++) sc[c][i] = -INFINITY;
+            continue;
+        }
+        if (c > 0) load(kv, kp, g.s_kn, c);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = d_ok ? fmaf(q4[e], kv[i][e], s) : 0.f;
+            s += dpp_f<DPP_QUAD_XOR1>(s);
+            s += dpp_f<DPP_QUAD_XOR2>(s);
+            s += dpp_f<DPP_ROW_HALF_MIRROR>(s);
+            if constexpr (LPR >= 16) s += dpp_f<DPP_ROW_MIRROR>(s);
+            if constexpr (LPR >= 32) s += __shfl_xor(s, 16);
+            sc[c][i] = c * DCH + i * KG + kg < n ? s : -INFINITY;
+            mloc = fmaxf(mloc, sc[c][i]);
+        }
     }
     float m = block_reduce4(mloc, MaxOp(), red);
     PITON_PHASE(2);
     const float mref = m == -INFINITY ? 0.f : m;  // a chunk of -inf scores alone: every weight 0
     float lsum = 0.f;
 #pragma unroll
-    for (int i = 0; i < NR; i++) {
-        sc[i] = __builtin_amdgcn_exp2f(sc[i] - mref);
-        lsum += sc[i];
-    }
-    if (n < DCH)
+    for (int c = 0; c < CH; c++)
 #pragma unroll
-        for (int i = 0; i < NR; i++)
-            if (i * KG + kg >= n) vv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < NR; i++) {
+            sc[c][i] = __builtin_amdgcn_exp2f(sc[c][i] - mref);
+            lsum += sc[c][i];
+        }
     // the lane group's part of P V, the weights times `scale`
     auto add_up = [&](float scale) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < NR; i++)
+        for (int c = 0; c < CH; c++) {
+            if (c > 0 && c * DCH >= n) continue;
+            if (CH > 1) load(vv, vp, g.s_vn, c);
+            if (n < (c + 1) * DCH)
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[e] = fmaf(sc[i] * scale, vv[i][e], acc[e]);
-        *reinterpret_cast<f32x4 *>(&part[kg][4 * dq]) = acc;
-        return fmaxf(fmaxf(fabsf(acc.x), fabsf(acc.y)), fmaxf(fabsf(acc.z), fabsf(acc.w)));
+                for (int i = 0; i < NR; i++)
+                    if (c * DCH + i * KG + kg >= n) vv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NR; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] = fmaf(sc[c][i] * scale, vv[i][e], acc[e]);
+            sum = c > 0 ? sum + acc : acc;
+        }
+        *reinterpret_cast<f32x4 *>(&part[kg][4 * dq]) = sum;
+        return fmaxf(fmaxf(fabsf(sum.x), fabsf(sum.y)), fmaxf(fabsf(sum.z), fabsf(sum.w)));
     };
-    if (add_up(1.f) >= 0x1p121f) large = 1;
+    if (add_up(1.f) >= 0x1p121f && SPLIT) large = 1;
     float l = block_reduce4(dq == 0 ? lsum : 0.f, SumOp(), red + 4);  // its barrier publishes the sums
     // values that take a chunk's sum near the largest float, which the whole softmax may give little
     // weight or none: the chunk leaves its sums 2^-9 as large under a maximum 9 higher
-    if (nsplit > 1 && large) {
+    if (SPLIT && large) {
         add_up(0x1p-9f);
         __syncthreads();
         m += 9.f;
@@ -1011,7 +1034,7 @@ void attn_decode_part(DecodeArgs g, float *ws, int nsplit) {
 #pragma unroll
         for (int w = 1; w < KG; w++) v += part[w][t];
     }
-    if (nsplit == 1) {
+    if constexpr (!SPLIT) {
         // (every score -inf: 0 / 0, NaN as the softmax of such a row is)
         if (t < D && t < g.head_dim) g.o[b * g.s_ob + h * g.s_oh + t] = v * (1.0f / l);
     } else {
@@ -1057,11 +1080,15 @@ __global__ __launch_bounds__(256) void attn_decode_merge(DecodeArgs g, const flo
     }
 }
 
-// The chunks of a decode attention call's cache; more than one needs a workspace of
-// decode_workspace() floats. Splitting wins at every head count measured: 8 heads x 4096 keys
-// 155 -> 9 us, 1024 heads x 512 keys (enough workgroups to fill the chip unsplit) 53 -> 46 us.
-static int decode_parts(int64_t n_keys, int32_t head_dim) {
+// The workgroups per head of a decode attention call; more than one need a workspace of
+// decode_workspace() floats. Splitting wins while the heads leave CUs without work: 8 heads x 4096
+// keys 155 -> 9 us, 384 heads x 258 keys of 64 14.0 -> 13.0. From two heads per CU on, up to three chunks in one
+// workgroup do: 512 heads x 258 keys of 64 15.9 -> 12.4 us, 1024 x 640 57.7 -> 52.1, 1024 x 517 keys of
+// 32 34.5 -> 28.2 (a workgroup over all keys in a chain, attn_decode_kernel: 15.4, 63.7, 24.7). Past
+// three, splitting again (1024 heads x 793 keys of 64 79.7 -> 71).
+static int decode_parts(int64_t n_keys, int64_t nbh, int32_t head_dim) {
     const int chunk = head_dim <= 32 ? kDecodeChunk<32> : head_dim == 64 ? kDecodeChunk<64> : kDecodeChunk<128>;
+    if (nbh >= 2 * (int64_t)device_cu_count() && n_keys <= 3 * chunk) return 1;
     return (int)((n_keys + chunk - 1) / chunk);
 }
 static int64_t decode_workspace(int64_t nbh, int parts, int32_t head_dim) {
@@ -1193,8 +1220,8 @@ int32_t piton_mi355x_attn_decode_workspace(int64_t n_keys, int64_t batch, int64_
     int rc = require_device();
     if (rc) return rc;
     if (n_keys >= 1 && n_keys <= kMaxDecodeKeys && batch > 0 && n_heads > 0) {
-        const int parts = decode_parts(n_keys, head_dim);
         const int64_t nbh = sat_mul(batch, n_heads);
+        const int parts = decode_parts(n_keys, nbh, head_dim);
         if (parts > 1 && sat_mul(nbh, parts) <= 0x7FFFFFFF) *floats = decode_workspace(nbh, parts, head_dim);
     }
     clear_error();
@@ -1225,28 +1252,33 @@ int32_t piton_mi355x_attn_decode_split(const float *q, const float *k, const flo
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)(batch * n_heads)), block(256);
     const bool vec = aligned16(k) && stride_kn % 4 == 0 && stride_kh % 4 == 0 && stride_kb % 4 == 0;
-    const int parts = decode_parts(n_keys, head_dim);
+    const int parts = decode_parts(n_keys, batch * n_heads, head_dim);
     if (parts == 1 || (workspace && sat_mul(batch * n_heads, parts) <= 0x7FFFFFFF &&
                        workspace_floats >= decode_workspace(batch * n_heads, parts, head_dim))) {
         const bool vec4 = vec && aligned16(v) && stride_vn % 4 == 0 && stride_vh % 4 == 0 && stride_vb % 4 == 0;
         const dim3 pgrid((unsigned)(batch * n_heads * parts));
-#define PITON_DEC_ROWS(D, NR)                                                                                       \
+#define PITON_DEC_ROWS(D, NR, CH)                                                                                   \
     do {                                                                                                            \
         if (vec4)                                                                                                   \
-            PITON_LAUNCH_NAMED((attn_decode_part<D, true, NR>), "attn_decode_part<" #D ", true, " #NR ">", pgrid,   \
-                               block, 0, st, g, workspace, parts);                                                  \
+            PITON_LAUNCH_NAMED((attn_decode_part<D, true, NR, CH>),                                                 \
+                               "attn_decode_part<" #D ", true, " #NR ", " #CH ">", pgrid, block, 0, st, g,          \
+                               workspace, parts);                                                                   \
         else                                                                                                        \
-            PITON_LAUNCH_NAMED((attn_decode_part<D, false, NR>), "attn_decode_part<" #D ", false, " #NR ">", pgrid, \
-                               block, 0, st, g, workspace, parts);                                                  \
+            PITON_LAUNCH_NAMED((attn_decode_part<D, false, NR, CH>),                                                \
+                               "attn_decode_part<" #D ", false, " #NR ", " #CH ">", pgrid, block, 0, st, g,         \
+                               workspace, parts);                                                                   \
     } while (0)
 #define PITON_DEC_SPLIT(D)                                                                                          \
     do {                                                                                                            \
         const int64_t rows = (n_keys + 1024 / D - 1) / (1024 / D); /* 1024 / D keys per row of a workgroup */       \
-        if (rows <= 1) PITON_DEC_ROWS(D, 1);                                                                        \
-        else if (rows <= 2) PITON_DEC_ROWS(D, 2);                                                                   \
-        else if (rows <= 4) PITON_DEC_ROWS(D, 4);                                                                   \
-        else if (rows <= 8) PITON_DEC_ROWS(D, 8);                                                                   \
-        else PITON_DEC_ROWS(D, 16);                                                                                 \
+        if (rows <= 1) PITON_DEC_ROWS(D, 1, 1);                                                                        \
+        else if (rows <= 2) PITON_DEC_ROWS(D, 2, 1);                                                                   \
+        else if (rows <= 4) PITON_DEC_ROWS(D, 4, 1);                                                                   \
+        else if (rows <= 8) PITON_DEC_ROWS(D, 8, 1);                                                                   \
+        else if (parts > 1) PITON_DEC_ROWS(D, 16, 0);                                                               \
+        else if (rows <= 16) PITON_DEC_ROWS(D, 16, 1);                                                              \
+        else if (rows <= 32) PITON_DEC_ROWS(D, 8, 4);                                                               \
+        else PITON_DEC_ROWS(D, 8, 6);                                                                               \
         if (parts > 1) PITON_LAUNCH((attn_decode_merge<D>), grid, block, 0, st, g, workspace, parts);               \
     } while (0)
         if (head_dim <= 32) PITON_DEC_SPLIT(32);

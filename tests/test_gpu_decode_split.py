@@ -88,6 +88,56 @@ def test_masked_and_infinite_keys():
     assert np.isposinf(got[0, 2, 7]) and np.isfinite(np.delete(got[0, 2], 7)).all()
 
 
+def _past_nan(B, H, n, dh, pad):
+    """A cache of n + 70 rows, the last 70 and the padding NaN, and float64's result over the first n."""
+    q, k, v = _cache(B, H, n + 70, dh, pad, dh + n + B)
+    ref = _fp64(q, k[:n], v[:n], 0.3)
+    for x in (k, v):
+        x[n:] = np.nan
+        x[..., dh:] = np.nan
+    tq, tk, tv = (torch.from_numpy(x).cuda() for x in (q, k, v))
+    out = torch.full((B + 1, H, dh), -9.0, device="cuda")
+    a = list(_args(tq, tk, tv, out, 0.3))
+    a[15] = n
+    rt.attn_decode(*a)
+    assert (out[B:] == -9.0).all()
+    return out[:B].cpu().numpy(), ref, [x["kernel"] for x in rt.last_launches()]
+
+
+@pytest.mark.parametrize("dh", [16, 32, 64, 128])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_every_row_count(dh, pad):
+    """One chunk: the kernels of 1, 2, 4, 8 and 16 rows per thread at the edges of their keys."""
+    per = 1024 // max(dh, 32)
+    for rows, kernel in ((1, 1), (2, 2), (3, 4), (4, 4), (5, 8), (8, 8), (9, 16), (16, 16)):
+        for n in sorted({(rows - 1) * per + 1, rows * per - 1, rows * per}):
+            got, ref, names = _past_nan(2, 3, n, dh, pad)
+            assert len(names) == 1 and f", {kernel}, 1>" in names[0], (n, names)
+            assert fp64.rel_fro(got, ref) <= 1e-5, n
+
+
+@pytest.mark.parametrize("dh", [32, 64, 128])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_many_heads_take_several_chunks_in_one_workgroup(dh, pad):
+    """Two heads per CU and more: up to three chunks' keys in one launch, four split as before."""
+    B, H, chunk = 2 * rt.device_info()["cu_count"] // 8, 8, 16384 // dh
+    g = torch.Generator(device="cuda").manual_seed(dh + pad)
+    q = torch.randn((B, H, dh), device="cuda", generator=g)
+    k, v = (torch.randn((3 * chunk + 2, B, H, dh + pad), device="cuda", generator=g) for _ in range(2))
+    out = torch.empty_like(q)
+    for n in (chunk + 1, chunk + chunk // 2, 2 * chunk, 2 * chunk + 1, 3 * chunk - 1, 3 * chunk, 3 * chunk + 1):
+        tail = k[n:].clone(), v[n:].clone()
+        k[n:], v[n:] = float("nan"), float("nan")
+        a = list(_args(q, k, v, out, 0.3))
+        a[15] = n
+        rt.attn_decode(*a)
+        assert len(rt.last_launches()) == (1 if n <= 3 * chunk else 2), n
+        k[n:], v[n:] = tail
+        p = torch.softmax((k[:n, ..., :dh].double() * q.double()).sum(-1) * 0.3, 0)
+        ref = (p[..., None] * v[:n, ..., :dh].double()).sum(0)
+        assert ((out.double() - ref).norm() / ref.norm()).item() <= 1e-5, n
+
+
 @pytest.mark.parametrize("dh,n", [(64, 600), (128, 300), (32, 1100)])
 def test_large_values_of_keys_without_weight(dh, n):
     """Finite values near the largest float whose keys have a weight of 0, or next to it, beside the
