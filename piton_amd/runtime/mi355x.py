@@ -11,6 +11,7 @@ on torch's current stream. A missing library or a failed call raises; there is n
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import struct
 import threading
@@ -356,24 +357,48 @@ def attn_decode(q, k, v, out, sm_scale, s_qb, s_qh, s_kb, s_kh, s_kn, s_vb, s_vh
     check_tensor("out", out, max_offset=_span((batch, s_ob), (heads, s_oh), (head_dim, 1)))
     args = (_ptr(q), _ptr(k), _ptr(v), _ptr(out), float(sm_scale), s_qb, s_qh, s_kb, s_kh, s_kn, s_vb, s_vh, s_vn, s_ob,
             s_oh, n_keys, batch, heads, int(head_dim))
-    # a cache of one chunk (16384 / head_dim keys) needs no workspace
-    ws = _decode_workspace(n_keys, batch, heads, int(head_dim)) if n_keys > 16384 // max(int(head_dim), 32) else None
+    ws = _decode_workspace(n_keys, batch, heads, int(head_dim)) if n_keys > _decode_chunk(int(head_dim)) else None
     if ws is None:
         _call("piton_mi355x_attn_decode", *args, _stream())
     else:
         _call("piton_mi355x_attn_decode_split", *args, _ptr(ws), ws.numel(), _stream())
 
 
+def _decode_floats(n_keys, batch, heads, head_dim) -> int:
+    """The floats of workspace that the library asks for; 0 where the call does not split."""
+    n = _i64(0)
+    _call("piton_mi355x_attn_decode_workspace", n_keys, batch, heads, head_dim, ctypes.byref(n))
+    return n.value
+
+
+@functools.lru_cache(maxsize=16)
+def _decode_chunk(head_dim) -> int:
+    """Keys up to which no call of this head_dim splits (one head is the first to): short caches need not
+    ask for a workspace, which takes 1 us of host time."""
+    hi = 1
+    while not _decode_floats(hi, 1, 1, head_dim):
+        hi *= 2
+        if hi > 1 << 30:
+            return hi  # never splits
+    lo = hi // 2
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        if _decode_floats(mid, 1, 1, head_dim):
+            hi = mid
+        else:
+            lo = mid
+    return lo
+
+
 def _decode_workspace(n_keys, batch, heads, head_dim):
     """The split decode attention's workspace, or None where the call does not split (or the
     device has no memory left for it: the unsplit kernel needs none)."""
-    n = _i64(0)
-    _call("piton_mi355x_attn_decode_workspace", n_keys, batch, heads, head_dim, ctypes.byref(n))
-    if n.value == 0:
+    floats = _decode_floats(n_keys, batch, heads, head_dim)
+    if floats == 0:
         return None
     try:
-        # (float32 whatever torch's default dtype is: n counts the kernels' floats)
-        return torch.empty(n.value, dtype=torch.float32, device="cuda")
+        # (float32 whatever torch's default dtype is: the kernels' floats are counted)
+        return torch.empty(floats, dtype=torch.float32, device="cuda")
     except torch.OutOfMemoryError:
         return None
 

@@ -218,6 +218,35 @@ def test_decode_workspace_is_float32_under_any_default_dtype(monkeypatch, dtype)
     assert ws is made[0] and ws.dtype == torch.float32 and ws.numel() * ws.element_size() == 4 * floats
 
 
+@pytest.mark.parametrize("chunk", [100, 256, 4096])
+def test_decode_asks_for_a_workspace_past_the_librarys_chunk(monkeypatch, chunk):
+    """Whatever the library's chunk of keys is, a cache past it takes the split entry with the floats
+    the library asks for, and one within it the plain entry."""
+    calls = []
+
+    def call(name, *args):
+        calls.append(name)
+        if name == "piton_mi355x_attn_decode_workspace":
+            n_keys = args[0]
+            args[-1]._obj.value = 7 * n_keys if chunk < n_keys <= 8192 else 0
+
+    monkeypatch.setattr(mi355x, "_call", call)
+    monkeypatch.setattr(mi355x, "check_tensor", lambda *a, **k: None)
+    monkeypatch.setattr(mi355x, "_stream", lambda: None)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: empty(*a, **{**k, "device": "cpu"}))
+    mi355x._decode_chunk.cache_clear()
+    try:
+        t = torch.zeros(4)
+        for n_keys in (1, chunk - 1, chunk, chunk + 1, 2 * chunk, 8192):
+            calls.clear()
+            mi355x.attn_decode(t, t, t, t, 1.0, *([0] * 10), n_keys, 1, 1, 64)
+            want = "piton_mi355x_attn_decode" + ("_split" if n_keys > chunk else "")
+            assert calls[-1] == want, (n_keys, calls)
+    finally:
+        mi355x._decode_chunk.cache_clear()
+
+
 # -- the reference-side hunks (INTEGRATION.md) driven on any host ------------------------------------
 
 @pytest.fixture

@@ -116,6 +116,13 @@ def test_every_row_count(dh, pad):
             assert fp64.rel_fro(got, ref) <= 1e-5, n
 
 
+@pytest.mark.parametrize("dh", [16, 32, 64, 128])
+def test_the_chunk_is_the_librarys(dh):
+    chunk = rt._decode_chunk(dh)
+    assert chunk == 16384 // max(dh, 32)
+    assert [rt._decode_floats(n, 2, 3, dh) > 0 for n in (1, chunk, chunk + 1, 8192, 8193)] == [0, 0, 1, 1, 0]
+
+
 @pytest.mark.parametrize("dh", [32, 64, 128])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_many_heads_take_several_chunks_in_one_workgroup(dh, pad):
