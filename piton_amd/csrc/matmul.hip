@@ -213,7 +213,8 @@ __device__ __forceinline__ void store_b(const GemmArgs &g, int t, float (&Bs)[GB
 constexpr int kStages = PITON_GEMM_STAGES;
 
 // FULL: row-major A and B, M and N multiples of 128 and K of 32, so every tile is interior and
-// every K tile whole. Without the guarded paths the kernel fits 128 registers and runs four
+// every K tile whole; only operands of 2^29 floats or more, past the offsets of the split and the
+// direct kernel, come here. Without the guarded paths the kernel fits 128 registers and runs four
 // workgroups per CU (4096^3: the 1024 tiles in one generation; 3 % faster than three per CU).
 // Layouts with a scalar (any-stride) loader need more registers: two workgroups per CU.
 template <int A_L, int B_L, bool FULL>
@@ -788,10 +789,11 @@ void gemm_split_kernel(GemmArgs g) {
             }
     };
     // this wave's K tiles: wave, wave + KS, ...; the next one is in flight while one multiplies.
-    // Tiles come in pairs with no condition between loads and products (a conditional product
-    // lets the compiler sink its loads next to it, ending the prefetch): a tile past the last
-    // one reads zeros for A (k >= K) and B (rows past K) and adds exact zeros; the prefetch
-    // after the last pair is never used.
+    // The loop takes whole passes of two tiles (four with four sums) with no condition between loads
+    // and products (a conditional product lets the compiler sink its loads next to it, ending the
+    // prefetch). TAIL takes the tiles that fill no pass, and the partial one, ahead of it; without
+    // TAIL a wave's last pass may hold a tile past the last one, which reads zeros and adds exact
+    // zeros. The prefetch after the last pass is never used.
     // The scheduling barriers keep each tile's loads together ahead of the other tile's products
     // (left free, the scheduler moves every load next to its first use to save registers).
     // Each half-step issues the next tile's loads between this tile's products, PITON_SPLIT_LPM

@@ -211,21 +211,24 @@ def test_decode_ignores_cache_rows_past_n_keys(n_keys):
     np.testing.assert_array_equal(got.view(np.uint32), exact.view(np.uint32))
 
 
-@pytest.mark.parametrize("dh", [32, 64])
-def test_short_and_long_decode_kernels_agree(dh):
-    """Caches of up to 256 keys take the kernel that requests all of K and V up front, longer ones
-    the chunked kernel; their arithmetic is the same. A 257th key whose score is -inf adds
-    exactly zero to the sum and to P V, so 257 keys on the long kernel give the bits of the
-    first 256 on the short one."""
+@pytest.mark.parametrize("dh,n", [(32, 256), (32, 512), (64, 256), (128, 128)])
+def test_a_masked_key_more_gives_the_same_bits(dh, n):
+    """One key more whose score is -inf adds exactly zero to the sum and to P V, so n + 1 keys give
+    the bits of the first n: within a chunk of 16384 / dh keys, and past one, where the last key is a
+    chunk of its own that the merge adds with a weight of zero."""
     rng = np.random.default_rng(dh)
     B, H = 3, 2
     q = np.abs(rng.standard_normal((B, H, dh))).astype(np.float32) + np.float32(0.1)
-    k = rng.standard_normal((B, H, 257, dh)).astype(np.float32)
-    v = rng.standard_normal((B, H, 257, dh)).astype(np.float32)
-    k[:, :, 256] = -np.inf  # positive q: the score is -inf
-    short = _decode(q, k[:, :, :256], v[:, :, :256], 256)
-    long_ = _decode(q, k, v, 257)
-    np.testing.assert_array_equal(short.view(np.uint32), long_.view(np.uint32))
+    k = rng.standard_normal((B, H, n + 1, dh)).astype(np.float32)
+    v = rng.standard_normal((B, H, n + 1, dh)).astype(np.float32)
+    k[:, :, n] = -np.inf  # positive q: the score is -inf
+    one = _decode(q, k[:, :, :n], v[:, :, :n], n)
+    names = [x["kernel"] for x in rt.last_launches()]
+    assert len(names) == 1 and names[0].startswith(f"attn_decode_part<{dh}, "), names
+    more = _decode(q, k, v, n + 1)
+    names = [x["kernel"].partition("<")[0] for x in rt.last_launches()]
+    assert names == (["attn_decode_part", "attn_decode_merge"] if n * dh == 16384 else ["attn_decode_part"]), names
+    np.testing.assert_array_equal(one.view(np.uint32), more.view(np.uint32))
 
 
 def _decode_layer_case(B, H, n_keys, pad, seed):
