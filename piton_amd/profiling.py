@@ -54,8 +54,8 @@ WORKLOADS = {
 # their launches, identified by kernel name and Grid_Size_X (work-items), with the number of
 # times a step runs each (the 4096^3 matmul: two launches of 256 tiles of 128 x 256, one per CU;
 # the split GEMM's template arguments are <row blocks, column blocks, waves splitting K, A's
-# layout (0: rows 16-byte aligned, 1: unaligned rows), B column-major, K % 32 != 0>; the ragged
-# shape runs 240 wide tiles of 64 x 128)
+# layout (0: rows 16-byte aligned, 1: unaligned rows), B column-major, tiles ahead of the K loop,
+# partial sums per wave>; the ragged shape runs 240 wide tiles of 64 x 128)
 LAUNCHES = {
     ("gemm_direct_kernel<true, true, false, 4>", 65536): ("matmul 4096^3", 2),
     ("gemm_split_kernel<1, 1, 4, 0, false, false, 1>", 65536): ("matmul 512^3", 1),
