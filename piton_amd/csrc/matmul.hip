@@ -1580,7 +1580,7 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
     // whole tiles that fill whole generations (or a part of the first by the time model) run on the
     // direct kernel, 1-2 % faster there than the split kernel's 64 x 128 tiles; a last generation
     // that is part full costs a whole one, and the split kernel's cut makes up for it
-    // (3072^3, 2.25 generations: 540 -> 433 us)
+    // (3072^3, 2.25 generations: 536 -> 458 us)
     const int64_t dgens = gens(dtiles);
     const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
     const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums) : SplitPlan{};
