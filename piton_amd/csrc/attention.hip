@@ -904,9 +904,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(DecodeArgs g) {
 // unnormalised in the caller's workspace and attn_decode_merge adds them. Where the heads fill the
 // chip, one workgroup takes up to three chunks' keys itself, eight rows at a time. Bound by HBM:
 // attn_decode_kernel's one workgroup per head is a serial chain of key loads (64 heads x 4096
-// keys of 64: 64 of 256 CUs, 160 us, 0.84 TB/s); the chunks fill the chip and each workgroup
-// requests its 64 KB of K and V before it uses any of it (25 us, 5.4 TB/s with the merge; 6.3
-// TB/s at 256 heads x 4000 keys).
+// keys of 64: 64 of 256 CUs, 160 us, 0.84 TB/s); the chunks fill the chip and a thread keeps up to 16
+// float4 in flight, K's rows and then, ahead of the maximum's reduction, all of V's (25 us, 5.4 TB/s with
+// the merge; 6.3 TB/s at 256 heads x 4000 keys, each byte of K and V fetched once).
 //   * D/4 consecutive lanes share a row of K or V, one float4 each, so that a wave's load covers
 //     whole cache lines (16 of a key's dims per lane in four loads, attn_decode_kernel's way,
 //     touches every line eight times: 33 us, and 46 with nontemporal loads);

@@ -249,8 +249,8 @@ def main():
     for nk in (96, 160):
         m = decode_phases(nk)
         print(f"| decode attention 64 x 4 heads x 64, {nk} keys | {int(m['waves'])} | {us(m['last_wave_start'])} | "
-              f"{us(m['first_data'])} (K, V in) | {us(m['wave_wait'])} | {us(m['end'])} | {us(m['gap_to_next'])} | "
-              f"per wave: scores and max {us(m['loop'])}, exp, sum, P V {us(m['merge'])} |")
+              f"{us(m['first_data'])} (first rows in) | {us(m['wave_wait'])} | {us(m['end'])} | {us(m['gap_to_next'])} | "
+              f"per wave: other rows, scores and max {us(m['loop'])}, exp, sum, P V {us(m['merge'])} |")
     print()
     print("| fused decode step, 64 x 4 heads x 64 | layernorm | projection (waves 0-5) | cache copies (waves 6, 7) | "
           "attention | last wave ends | gap to next launch |")
