@@ -1362,7 +1362,7 @@ static int best_form(int64_t M, int64_t N, int64_t K, int layout, int cus, int l
 
 // A product as one launch, or as two: whole rounds of one form over the first rows (columns) of C
 // and the rest in the form that suits it, where the model finds that faster than letting a last
-// round run part full (2560^3 296 -> 269 us, 300 x 4000 x 3000 99.9 -> 68.4). parts 0: the split
+// round run part full (2560^3 299 -> 268 us, 300 x 4000 x 3000 99.5 -> 70.0). parts 0: the split
 // kernel does not apply. The cut and the partial sums depend on the sizes alone, and so does `us`, the
 // time that launch_gemm holds against the direct kernel's: every layout of A and B (and every group
 // order) of one of the two kernels adds each element's products in the same order and gives the same
@@ -1579,8 +1579,8 @@ static int launch_gemm(GemmArgs g, hipStream_t st, const char *what, int sums) {
     const int64_t dtiles = wide ? wtiles : ntiles;
     // whole tiles that fill whole generations (or a part of the first by the time model) run on the
     // direct kernel, 1-2 % faster there than the split kernel's 64 x 128 tiles; a last generation
-    // that is part full costs a whole one, and the split kernel's cut makes up for it
-    // (3072^3, 2.25 generations: 536 -> 458 us)
+    // that is part full costs a whole one, which the split kernel's smaller tiles and
+    // cuts save (3072^3, 2.25 generations: 541 -> 462 us)
     const int64_t dgens = gens(dtiles);
     const bool full_gens = direct && ntiles >= cus && dtiles % cus == 0;
     const SplitPlan sp = sums || !full_gens ? plan_split(g, cus, sums) : SplitPlan{};
